@@ -905,11 +905,16 @@ __device__ __forceinline__ uint32_t ffbh32(uint32_t a) {
   asm("v_ffbh_u32 %0, %1" : "=v"(r) : "v"(a));
   return r;
 }
-// min(a, b, 64) as one v_min3_u32 (kept whole: the compiler would otherwise move the 64
-// out of the two branches that compute a lifted length)
-__device__ __forceinline__ uint32_t min3_64(uint32_t a, uint32_t b) {
+// min(a, b, c) as one v_min3_u32 (kept whole: the compiler would otherwise move the last
+// minimum out of the two branches that compute a lifted length)
+__device__ __forceinline__ uint32_t min3u(uint32_t a, uint32_t b, uint32_t c) {
   uint32_t r;
-  asm("v_min3_u32 %0, %1, %2, 64" : "=v"(r) : "v"(a), "v"(b));
+  asm("v_min3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
+  return r;
+}
+__device__ __forceinline__ uint32_t min3v(uint32_t a, uint32_t b, uint32_t c) {
+  uint32_t r;
+  asm("v_min3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
 __device__ __forceinline__ int getbit(const uint32_t *w, int pos) { return (w[pos >> 5] >> (pos & 31)) & 1; }
@@ -1001,13 +1006,14 @@ constexpr int kCredCounters = 64;  // work counters of the balanced kernel: entr
 // the one-mismatch sets it enumerates, which is large on streams with long runs: many
 // positions with a short best match but thousands of one-mismatch candidates, or long
 // matches with long extension chains. The per-candidate path costs about the same per
-// candidate whatever the stream. Measured per position on random and trained-model
-// streams (T 2048), the per-candidate path is the cheaper one when a stream's mean best
-// length exceeds 12 or more than 40% of its positions have a best length below 8, and at
-// every position below 768 (a scan's cost grows with t, the bit-parallel path's hardly).
-constexpr int kScanBelow = 768;
+// candidate whatever the stream. The line was swept on B 4, T 2048, S 512: with mean best
+// lengths above 11, more than 30% of the positions below 8, or positions below 1024 on the
+// per-candidate path, the backward takes 5.16 / 5.85 / 5.97 ms on random streams and on
+// streams biased by 1 and 3 sigma (all positions per-candidate: 5.84 / 5.89 / 5.88; with 12,
+// 40% and 768: 5.16 / 5.88 / 6.11). A scan's cost grows with t, the bit-parallel path's hardly.
+constexpr int kScanBelow = 1024;
 __device__ __forceinline__ bool cred_scan_stream(int64_t len_sum, int64_t short_cnt, int T) {
-  return len_sum > 12 * (int64_t)T || 10 * short_cnt > 4 * (int64_t)T;
+  return len_sum > 11 * (int64_t)T || 10 * short_cnt > 3 * (int64_t)T;
 }
 
 // One block per stream: mode, zeroed sums and d loss / d payload = sum over t of
@@ -1153,11 +1159,25 @@ __device__ __forceinline__ void near_flips_tables(int lane, int t, int lmax, int
                                                   float g, long long gi, const CredAcc &ca, int T,
                                                   uint32_t *tab);
 __device__ __forceinline__ uint32_t wave_prefix_max(uint32_t v);
+// wave maximum, wave-uniform: rows of 16 by DPP, the four rows on the scalar unit
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = group_max_u32<16>(v);
+  const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16),
+                 c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+  uint32_t ab, cd, r;
+  asm("s_max_u32 %0, %1, %2" : "=s"(ab) : "s"(a), "s"(b) : "scc");
+  asm("s_max_u32 %0, %1, %2" : "=s"(cd) : "s"(c), "s"(d) : "scc");
+  asm("s_max_u32 %0, %1, %2" : "=s"(r) : "s"(ab), "s"(cd) : "scc");
+  return r;
+}
 
 // The per-candidate path for one position t, all lanes of the wave: every candidate's
 // common-suffix length from its 64-bit window, 64 candidates per step from the latest down,
 // into the bucket tables (Mw: best key per common-suffix bucket, Nw: per bucket after the
-// q flip at the first mismatch) and the k-extension events Rk; the flips inside the best
+// q flip at the first mismatch) and the k-extension events Rk. Bound by VALU issue and by the
+// steps' LDS round trips: the steps that cannot change Mw, the far best or an event only form
+// c, the lifted length and one compare with Nw (B 4, T 2048, S 512, every position here:
+// backward 6.09 -> 5.63 ms on runs of mean length 10, 6.42 -> 5.88 on strongly biased bits); the flips inside the best
 // run from near_flips_tables (tab: 256 words). Writes every table it reads first.
 __device__ __forceinline__ void scan_position(int lane, int t, int T, int lmax, uint64_t qwin, uint32_t best,
                                               int jstar, int cstar, int capstar, float sgn, float g,
@@ -1170,10 +1190,21 @@ __device__ __forceinline__ void scan_position(int lane, int t, int T, int lmax, 
   const int trunc_hi = jstar;
   const int near0 = jstar - 63;  // the near candidates: j in [near0 + 1, near0 + 125]
 
-  Mw[lane] = Nw[lane] = 0u;
-  if (lane == 0) Mw[64] = Nw[64] = 0u;
+  // buckets past the q flips' range take no key: their bound is never beaten
+  const int imax = min(min(Lstar, lmax - 1), t);
+  Mw[lane] = 0u;
+  Nw[lane] = lane > imax ? ~0u : 0u;
+  if (lane == 0) {
+    Mw[64] = 0u;
+    Nw[64] = ~0u;
+  }
   Rk[lane] = Rk[lane + 64] = 0u;
   uint32_t farbest = 0u;  // best key among j outside [j* - 62, j* + 62] (this lane's j)
+  // The longest far length so far (wave-uniform). Later candidates come first, so a candidate
+  // no longer than it changes neither the far best nor the latest j of any length: Mw and
+  // farbest are only touched in the few steps that hold a longer one.
+  int bound = 0;
+  int pend = 0;  // steps whose events may still be incomplete
 
   // candidates from the latest down, 64 per step (lane l: j = j0 + l): a bucket's best key is
   // its latest j, so the bucket tables are written only when a key beats the stored one.
@@ -1191,7 +1222,10 @@ __device__ __forceinline__ void scan_position(int lane, int t, int T, int lmax, 
     constexpr bool TOP = decltype(top_c)::value, LOW = decltype(low_c)::value;
     constexpr int NEAR = decltype(near_c)::value;
     const int jp1 = (j0 + 1) + lane;  // j + 1, the key's low half
-    if (!TOP || jp1 <= t) {
+    const bool in = !TOP || jp1 <= t;
+    uint64_t longer = 0, event = 0;
+    int c = 0;
+    if (in) {
       typedef __attribute__((address_space(3))) const uint32_t lds_u32;
       const uint32_t ka = kaddr + (uint32_t)(j0 >> 5) * 4u;
       const uint32_t wa = *(lds_u32 *)(uintptr_t)ka, wb = *(lds_u32 *)(uintptr_t)(ka + 4u),
@@ -1203,42 +1237,53 @@ __device__ __forceinline__ void scan_position(int lane, int t, int T, int lmax, 
       // count + 32 saturates and the min with 64 covers x = 0
       const uint32_t xh = (uint32_t)(x >> 32);
       const uint32_t lo32 = __builtin_elementwise_add_sat(ffbh32((uint32_t)x), 32u);
-      const int c = (int)min(min(ffbh32(xh), lo32), 64u);
-      const int cap = LOW ? min(jp1, lmax) : lmax;  // j >= 64 > lmax - 1 above the last step
-      const uint32_t key = ((uint32_t)min(c, cap) << 16) | (uint32_t)jp1;
-      if (key > Mw[c]) atomicMax(Mw + c, key);
-      const bool near_step = NEAR == 2 ? (j0 + 63 > near0 && j0 < near0 + 126) : NEAR == 1;
-      if (near_step) {
-        if ((unsigned)(jp1 - near0 - 2) > 124u) farbest = max(farbest, key);
-      } else {
-        farbest = max(farbest, key);
-      }
+      const uint32_t hi32 = ffbh32(xh);
+      const uint32_t cap = LOW ? (uint32_t)min(jp1, lmax) : (uint32_t)lmax;  // j >= 64 > lmax - 1 above
       // the key after flipping the q bit at j's first mismatch (x's top set bit): the
       // common suffix c + 1 + e once that mismatch is gone. With c >= cap the flipped bit
       // lies past the cap and nkey == key; with c = 64 (x = 0, shift taken mod 64) nkey has
-      // length 0: it then only reaches Nw[64], which no flip reads.
+      // length 0: it then only reaches Nw[64], which takes nothing.
       // When every lane's first mismatch lies in the window's high word (the common case),
       // the flip leaves the low word as it is, and its leading-zero count is shared with c's.
-      int nlen;
-      if (__all(c < 32)) {
-        nlen = (int)min3_64(ffbh32(xh ^ (0x80000000u >> c)), lo32);
+      uint32_t nlen;
+      if (__all(hi32 < 32u)) {
+        c = (int)hi32;
+        nlen = LOW ? min3v(ffbh32(xh ^ (0x80000000u >> c)), lo32, cap) : min3u(ffbh32(xh ^ (0x80000000u >> c)), lo32, (uint32_t)lmax);
       } else {
+        c = (int)min3u(hi32, lo32, 64u);
         const uint64_t xb = x ^ (0x8000000000000000ull >> (c & 63));
-        nlen = (int)min3_64(ffbh32((uint32_t)(xb >> 32)),
-                            __builtin_elementwise_add_sat(ffbh32((uint32_t)xb), 32u));
+        const uint32_t nh = ffbh32((uint32_t)(xb >> 32)), nl = __builtin_elementwise_add_sat(ffbh32((uint32_t)xb), 32u);
+        nlen = LOW ? min3v(nh, nl, cap) : min3u(nh, nl, (uint32_t)lmax);
       }
-      const uint32_t nkey = ((uint32_t)min(nlen, cap) << 16) | (uint32_t)jp1;
+      const uint32_t nkey = (nlen << 16) | (uint32_t)jp1;
+      longer = __ballot(c > bound);
       // (a) flipping k[j - c] extends j past the best (never for c >= cap: nkey == key)
-      if (__builtin_expect(nkey > best, 0)) {
+      event = __ballot(nkey > best);
+      if (nkey > Nw[c]) atomicMax(Nw + c, nkey);
+      if (event != 0 && nkey > best) {
         int p = jp1 - c;
         asm volatile("" : "+v"(p));
         p -= 1;
         if (!(p >= trunc_lo && p <= trunc_hi)) atomicMax(Rk + (p & 127), nkey);
       }
-      if (nkey > Nw[c]) atomicMax(Nw + c, nkey);
+    }
+    if constexpr (TOP) {  // set under a lane condition that lane 0 meets: wave-uniform again
+      longer = (uint32_t)__builtin_amdgcn_readfirstlane(longer != 0);
+      event = (uint32_t)__builtin_amdgcn_readfirstlane(event != 0);
+    }
+    if (longer != 0) {
+      const int cap = LOW ? min(jp1, lmax) : lmax;
+      uint32_t key = ((uint32_t)min(c, cap) << 16) | (uint32_t)jp1;
+      if (in && c > bound) atomicMax(Mw + c, key);
+      if (NEAR != 0 && (unsigned)(jp1 - near0 - 2) <= 124u) key = 0u;  // a near candidate
+      if (in) farbest = max(farbest, key);
+      const int f = (int)(wave_max(farbest) >> 16);
+      bound = f >= lmax ? 64 : f;
     }
     // events of p come from j in [p, p + 61]: every p >= j0 is now complete (below t)
-    {
+    if (event != 0) pend = 2;
+    if (pend != 0) {
+      pend = __builtin_amdgcn_readfirstlane(pend - 1);
       const int p = j0 + lane;
       if (!TOP || p < t) {
         uint32_t *slot = Rk + (j0 & 64) + lane;  // slot p mod 128 (j0 is a multiple of 64)
@@ -1259,40 +1304,36 @@ __device__ __forceinline__ void scan_position(int lane, int t, int T, int lmax, 
   using T_ = std::true_type;
   using N0 = std::integral_constant<int, 0>;
   using N1 = std::integral_constant<int, 1>;
-  using N2 = std::integral_constant<int, 2>;
   const int jtop = ((t - 1) / 64) * 64;
   if (jtop == 0) {
-    cand_step(0, T_{}, T_{}, N2{});
+    cand_step(0, T_{}, T_{}, N1{});
   } else {
-    cand_step(jtop, T_{}, F_{}, N2{});
+    cand_step(jtop, T_{}, F_{}, N1{});
     // the middle steps in three runs: above the near range, the (at most three) steps that
     // may reach it, and below it
     int j0 = jtop - 64;
     for (; j0 >= 64 && j0 >= near0 + 126; j0 -= 64) cand_step(j0, F_{}, F_{}, N0{});
     for (; j0 >= 64 && j0 + 63 > near0; j0 -= 64) cand_step(j0, F_{}, F_{}, N1{});
     for (; j0 >= 64; j0 -= 64) cand_step(j0, F_{}, F_{}, N0{});
-    cand_step(0, F_{}, T_{}, N2{});
+    cand_step(0, F_{}, T_{}, N1{});
   }
   // (farbest stays per lane: near_flips_tables takes the wave maximum of its own terms)
 
   // v: the endpoint's successor bit
   if (lane == 0 && Lstar >= 1) ca.add(2 * T + jstar + 1, sgn < 0.0f, g, gi);
 
-  // q: flip of q[t - i], one lane per i in [0, min(L*, lmax - 1)]. Lane c holds bucket c;
-  // g1 = max key over buckets < i (exclusive prefix scan), sj = latest j over buckets > i
-  // (exclusive suffix scan).
+  // q: flip of q[t - i], lane i in [0, imax]: bucket i's best lifted key, and the latest j
+  // with c > i at length i, a suffix maximum of Mw (a prefix one over the reversed table,
+  // turned back by one shuffle; j + 1 is a key's low half, 0 for an empty bucket; buckets 63
+  // and 64 pooled, as i <= 62). A candidate with c < i never decides: j* itself keeps length i
+  // when c* > i and lifts when c* = i (i <= L* <= c*).
   {
-    // DPP prefix maxima; the suffix one over the reversed table, turned back by one shuffle
-    // (j + 1 is a key's low half, 0 for an empty bucket)
-    // buckets 63 and 64 pooled: a q flip at offset i <= 62 only asks for c < i or c > i
-    const uint32_t g1 = wave_prefix_max(lane >= 1 ? Mw[lane - 1] : 0u);  // buckets < lane
     const uint32_t mr = lane == 1 ? max(Mw[63], Mw[64]) : Mw[64 - lane];
     const uint32_t sr = wave_prefix_max(lane >= 1 ? (mr & 0xffffu) : 0u);
     const int sj = (int)(uint32_t)__shfl((int)sr, 63 - lane) - 1;        // buckets > lane
-    const int imax = min(min(Lstar, lmax - 1), t);
     if (lane <= imax) {
       const int i = lane;
-      uint32_t nb = max(g1, Nw[i]);  // Nw[i]: the candidates with c == i, bit flipped
+      uint32_t nb = Nw[i];  // the candidates with c == i, bit flipped
       if (lane < 63 && sj >= 0) nb = max(nb, mkkey(min(i, min(sj + 1, lmax)), sj));
       const float s2 = sign_of(nb, vw);
       if (s2 != sgn) ca.add(t - i, s2 > 0.0f, g, gi);
