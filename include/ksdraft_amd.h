@@ -128,7 +128,8 @@ int ksd_quantize_dual(const void *x, int x_dtype, int64_t R, int64_t C, int grou
  * in one launch: a linear layer's fp32 weight and its input when both are quantized for a
  * training forward (reference ksdraft/kernels/linear.py:46-56 and :69 with the X^T recipe of
  * ks3_int8.py:417-420). The outputs are those of two ksd_quantize_dual calls; shapes the
- * fused kernel does not take (C % 8 != 0, unaligned rows) run as two calls. Group 128.
+ * fused kernel does not take (empty, or rows past its 32-bit offsets) run as two calls.
+ * Group 128.
  */
 int ksd_quantize_dual2(const void *x0, int64_t R0, int64_t C0, int8_t *codes0, uint16_t *scales0,
                        int8_t *codes_t0, uint16_t *scales_t0, const void *x1, int64_t R1,
@@ -141,7 +142,7 @@ int ksd_quantize_dual2(const void *x0, int64_t R0, int64_t C0, int8_t *codes0, u
  * Each 128-row tile sums its column in four 32-row parts ((p0 + p1) + (p2 + p3)); the tiles'
  * sums are added in tile order (an fp32 sum in another order than torch's: TOL).
  *   colsum     (C,) fp32
- *   workspace  fp32 scratch of ceil(R/128) * C * 4 bytes; R > 0, C % 8 == 0, aligned rows
+ *   workspace  fp32 scratch of ceil(R/128) * C * 4 bytes; R > 0
  */
 int ksd_quantize_dual_colsum(const void *x, int x_dtype, int64_t R, int64_t C, int group,
                              int8_t *codes, uint16_t *scales, int8_t *codes_t, uint16_t *scales_t,
@@ -170,9 +171,9 @@ int ksd_ce_row_stats(const float *logits, int64_t R, int64_t C, const int64_t *t
  * d mean-CE divided by the counted-row count). codes/scales and codes_t/scales_t are
  * exactly ksd_quantize_dual(dY, t_from_codes = 0) of these dY values. No reference
  * counterpart as one call (the reference's autograd materialises dY in fp32).
- *   group 128; dy_out (R, C) fp32 optional: when given, dY is also written there. Shapes
- *   with C % 8 != 0 (or unaligned buffers) require dy_out, which then serves as the
- *   staging buffer of the two-pass path.
+ *   group 128; dy_out (R, C) fp32 optional: when given, dY is also written there. Tensors
+ *   past the tile kernel's 32-bit offsets (R > 65535 * 128 or C > 2^22 - 1) require dy_out,
+ *   which then serves as the staging buffer of the two-pass path.
  */
 int ksd_ce_backward_quant_dual(const float *logits, int64_t R, int64_t C, const float *row_max,
                                const float *row_inv_sum, const int64_t *targets,
@@ -280,6 +281,18 @@ int ksd_w8a8_gemm_nt(const int8_t *a, const uint16_t *a_scales, const int8_t *w,
  *   workspace  16-byte aligned fp32 scratch of at least S*M*N*4 bytes (unused when S = 1)
  */
 int ksd_w8a8_gemm_splits(int64_t M, int64_t N, int64_t K, int group, int *splits);
+
+/*
+ * The zero padding of a GEMM's code operands along K (reference ksdraft/kernels/gemm.py:71-73),
+ * up to four operands in one launch: dst (rows, Kp) = src (rows, K) with Kp - K zeros per row.
+ *   Kp a multiple of 16, Kp >= K; dst 16-byte aligned, src rows of any alignment; n <= 4
+ */
+typedef struct KsdPadOperand {
+  const int8_t *src;
+  int8_t *dst;
+  int64_t rows, K, Kp;
+} KsdPadOperand;
+int ksd_pad_codes(const KsdPadOperand *list, int n, void *stream);
 /*
  * The general entry: split K as above, plus an optional residual operand added in the
  * store (the residual adds of reference ksdraft/model/block.py:39-41, h = x + linear(...)):

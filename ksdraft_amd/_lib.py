@@ -46,6 +46,7 @@ SIGNATURES = {
     "ksd_embedding_gather_int8": [_P, _P, _P, _I64, _I64, _I64, _INT, _P, _INT, _P],
     "ksd_w8a8_gemm_nt": [_P, _P, _P, _P, _I64, _I64, _I64, _INT, _P, _P, _INT, _P],
     "ksd_w8a8_gemm_splits": [_I64, _I64, _I64, _INT, _P],
+    "ksd_pad_codes": [_P, _INT, _P],
     "ksd_w8a8_gemm_nt_ws": [_P, _P, _P, _P, _I64, _I64, _I64, _INT, _P, _P, _INT, _P, _I64, _P],
     "ksd_w8a8_gemm_nt_ex": [_P, _P, _P, _P, _I64, _I64, _I64, _INT, _P, _P, _P, _INT, _P, _I64, _P],
     "ksd_w8a8_gemm_pair": [_P, _P, _P, _P, _I64, _I64, _I64, _P, _INT, _P, _P, _P, _P, _I64, _I64, _I64,

@@ -290,8 +290,7 @@ __global__ __launch_bounds__(256) void requant_T_multi_kernel(const RqtBatchArg 
 // kernel, quant_dual_codes_kernel, below. The rows are
 // quantized from registers (16 lanes per row, 8 elements each), the values then go to LDS
 // transposed in quant_T_kernel's conflict-free layout, and 4 lanes per column quantize the
-// columns. Requires C % 8 == 0 and 16-byte aligned rows; rows past R read as zeros and
-// are not stored.
+// columns. Rows past R read as zeros and are not stored.
 // Cross-entropy backward source of the dual kernel: x[r, c] is not read from memory but
 // formed from fp32 logits y and per-row softmax statistics,
 //   dY[r, c] = (exp(y[r, c] - max_r) / sum_r - [c == t_r]) * w_r,
@@ -305,12 +304,42 @@ struct CeSrc {
 };
 constexpr float kLog2e = 1.4426950408889634f;
 
+// The 8 elements of a row from column col on, zeros past C: rows of any length and alignment
+// (unaligned 16-byte loads inside the row, single elements at its end).
+template <int DT>
+__device__ __forceinline__ void load_ragged8(const typename Elem<DT>::T *row, int64_t col, int64_t C, bool ok, float *v) {
+  typename Elem<DT>::T e[8] = {};
+  if (ok && col + 8 <= C) {
+    __builtin_memcpy(e, row + col, sizeof(e));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (ok && col + i < C) e[i] = row[col + i];
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = Elem<DT>::load(e + i);
+}
+// Their 8 codes (two packed words).
+__device__ __forceinline__ void store_ragged8(const uint32_t *w, int8_t *row, int64_t col, int64_t C, bool ok) {
+  if (ok && col + 8 <= C) {
+    __builtin_memcpy(row + col, w, 8);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (ok && col + i < C) row[col + i] = (int8_t)(w[i >> 2] >> (8 * (i & 3)));
+  }
+}
+
+// VEC: C % 8 == 0 and 16-byte aligned rows. Otherwise rows go through the ragged helpers: one
+// pass over x either way, where ragged rows took a row kernel, a transposing kernel and, for
+// the column sums, two torch kernels. A ragged gradient (509 x 777 bf16, codes, transposed codes and
+// sums) takes 15 us of kernels in two launches.
 // col_part (optional, not with CE): (ceil(R/128), C) fp32 partial column sums of x, one row
 // per 128-row tile, each the sum of its four 32-row parts ((p0 + p1) + (p2 + p3)), every
 // part summed in row order; colsum_finalize_kernel adds the tiles in order.
 // H16: quantize the fp16 rounding of x (x.to(float16) first: the KS3 cell's backward
 // quantizes its upstream gradient as g16 = grad.to(float16), ks3_int8.py:345-348, :421-422).
-template <int DT, bool CE = false, bool H16 = false>
+template <int DT, bool CE = false, bool H16 = false, bool VEC = true>
 __global__ __launch_bounds__(512) void quant_dual_kernel(
     const void *__restrict__ xv, int64_t R, int64_t C, int8_t *__restrict__ codes,
     uint16_t *__restrict__ scales, int8_t *__restrict__ codes_t, uint16_t *__restrict__ scales_t,
@@ -333,17 +362,20 @@ __global__ __launch_bounds__(512) void quant_dual_kernel(
   const int rr = tid >> 4, sub = tid & 15;
   const int64_t col = c0 + sub * 8;
   const bool cok = col < C;
-  const T *xb = (const T *)xv + (cok ? col : 0);
+  const T *xb = (const T *)xv + (VEC && cok ? col : 0);
   Raw8<DT> raw[4];
+  if constexpr (VEC) {
 #pragma unroll
-  for (int p = 0; p < 4; ++p) raw[p] = load_raw8<DT>(xb + min(r0 + 32 * p + rr, R - 1) * C);
+    for (int p = 0; p < 4; ++p) raw[p] = load_raw8<DT>(xb + min(r0 + 32 * p + rr, R - 1) * C);
+  }
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     const int lr = 32 * p + rr;  // row within the tile
     const int64_t row = r0 + lr;
     const bool ok = cok && row < R;
     float v[8];
-    cvt_raw8<DT>(raw[p], ok, v);
+    if constexpr (VEC) cvt_raw8<DT>(raw[p], ok, v);
+    else load_ragged8<DT>(xb + min(row, R - 1) * C, col, C, ok, v);
     if constexpr (H16) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] = f16_round(v[i]);
@@ -356,9 +388,14 @@ __global__ __launch_bounds__(512) void quant_dual_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float e = __builtin_amdgcn_exp2f((v[i] - m) * kLog2e) * inv;
-        v[i] = live ? (e - (col + i == t ? 1.0f : 0.0f)) * w : 0.0f;
+        v[i] = live && (VEC || col + i < C) ? (e - (col + i == t ? 1.0f : 0.0f)) * w : 0.0f;
       }
-      if (ce.dy) {
+      if (!VEC && ce.dy) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (ok && col + i < C) ce.dy[row * C + col + i] = v[i];
+      }
+      if (VEC && ce.dy) {
         typedef float f32x4 __attribute__((ext_vector_type(4)));
         typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
         const auto dr = rsrc(ce.dy + r0 * C, 4 * nrows * C);
@@ -376,7 +413,8 @@ __global__ __launch_bounds__(512) void quant_dual_kernel(
     u32x2 q;
     q.x = w[0];
     q.y = w[1];
-    __builtin_amdgcn_raw_buffer_store_b64(q, rq, ok ? (uint32_t)(lr * C + col) : kOob, 0, 0);
+    if constexpr (VEC) __builtin_amdgcn_raw_buffer_store_b64(q, rq, ok ? (uint32_t)(lr * C + col) : kOob, 0, 0);
+    else store_ragged8(w, codes + row * C, col, C, ok);
     __builtin_amdgcn_raw_buffer_store_b16(scale_bits(s), rs,
                                           ok && sub == 0 ? (uint32_t)(lr * ngC + col / G) * 2 : kOob, 0, 0);
 #pragma unroll
@@ -442,7 +480,7 @@ __global__ __launch_bounds__(256) void colsum_finalize_kernel(const float *__res
 // bank conflicts on the byte writes and the dword reads), and the 128 row scales; 17.4 KB
 // instead of 74 KB, so four blocks fit a CU. The column pass dequantizes code * scale
 // (exact in fp32, as in quant_dual_kernel) before its amax and codes.
-template <int DT>
+template <int DT, bool VEC>
 __device__ __forceinline__ void dual_codes_tile(
     const void *__restrict__ xv, int64_t R, int64_t C, int8_t *__restrict__ codes,
     uint16_t *__restrict__ scales, int8_t *__restrict__ codes_t, uint16_t *__restrict__ scales_t,
@@ -462,17 +500,20 @@ __device__ __forceinline__ void dual_codes_tile(
   const int rr = tid >> 4, sub = tid & 15;
   const int64_t col = c0 + sub * 8;
   const bool cok = col < C;
-  const T *xb = (const T *)xv + (cok ? col : 0);
+  const T *xb = (const T *)xv + (VEC && cok ? col : 0);
   Raw8<DT> raw[4];
+  if constexpr (VEC) {
 #pragma unroll
-  for (int p = 0; p < 4; ++p) raw[p] = load_raw8<DT>(xb + min(r0 + 32 * p + rr, R - 1) * C);
+    for (int p = 0; p < 4; ++p) raw[p] = load_raw8<DT>(xb + min(r0 + 32 * p + rr, R - 1) * C);
+  }
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     const int lr = 32 * p + rr;
     const int64_t row = r0 + lr;
     const bool ok = cok && row < R;
     float v[8];
-    cvt_raw8<DT>(raw[p], ok, v);
+    if constexpr (VEC) cvt_raw8<DT>(raw[p], ok, v);
+    else load_ragged8<DT>(xb + min(row, R - 1) * C, col, C, ok, v);
     const uint32_t am = group_max_u32<16>(__builtin_bit_cast(uint32_t, abs_max<8>(v)));
     const float s = group_scale(__builtin_bit_cast(float, am));
     uint32_t w[2];
@@ -481,7 +522,8 @@ __device__ __forceinline__ void dual_codes_tile(
     u32x2 q;
     q.x = w[0];
     q.y = w[1];
-    __builtin_amdgcn_raw_buffer_store_b64(q, rq, ok ? (uint32_t)(lr * C + col) : kOob, 0, 0);
+    if constexpr (VEC) __builtin_amdgcn_raw_buffer_store_b64(q, rq, ok ? (uint32_t)(lr * C + col) : kOob, 0, 0);
+    else store_ragged8(w, codes + row * C, col, C, ok);
     __builtin_amdgcn_raw_buffer_store_b16(scale_bits(s), rs,
                                           ok && sub == 0 ? (uint32_t)(lr * ngC + col / G) * 2 : kOob, 0, 0);
 #pragma unroll
@@ -523,11 +565,11 @@ __device__ __forceinline__ void dual_codes_tile(
   }
 }
 
-template <int DT>
+template <int DT, bool VEC>
 __global__ __launch_bounds__(512) void quant_dual_codes_kernel(
     const void *__restrict__ xv, int64_t R, int64_t C, int8_t *__restrict__ codes,
     uint16_t *__restrict__ scales, int8_t *__restrict__ codes_t, uint16_t *__restrict__ scales_t) {
-  dual_codes_tile<DT>(xv, R, C, codes, scales, codes_t, scales_t, blockIdx.x, blockIdx.y);
+  dual_codes_tile<DT, VEC>(xv, R, C, codes, scales, codes_t, scales_t, blockIdx.x, blockIdx.y);
 }
 
 // Two X operands (e.g. a layer's weight and its input) in one launch: blocks
@@ -541,13 +583,13 @@ struct DualOperand {
   int8_t *codes_t;
   uint16_t *scales_t;
 };
-template <int DT>
+template <int DT, bool VEC>
 __global__ __launch_bounds__(512) void quant_dual_codes2_kernel(DualOperand a, DualOperand b) {
   const int64_t ta = ((a.C + 127) / 128) * ((a.R + 127) / 128);
   const int64_t i = blockIdx.x;
   const DualOperand &o = i < ta ? a : b;
   const int64_t j = i < ta ? i : i - ta, tc = (o.C + 127) / 128;
-  dual_codes_tile<DT>(o.x, o.R, o.C, o.codes, o.scales, o.codes_t, o.scales_t, j % tc, j / tc);
+  dual_codes_tile<DT, VEC>(o.x, o.R, o.C, o.codes, o.scales, o.codes_t, o.scales_t, j % tc, j / tc);
 }
 
 // ---------------------------------------------------------------- cross entropy
@@ -1100,10 +1142,9 @@ extern "C" int ksd_quantize_dual(const void *x, int x_dtype, int64_t R, int64_t 
   if (t_from_codes < 0 || t_from_codes > 2) return fail(KSD_EINVAL, "quantize_dual: mode must be 0, 1 or 2");
   hipStream_t st = (hipStream_t)stream;
   const int esz = x_dtype == KSD_F32 ? 4 : 2;
-  const bool fast = group == 128 && C % 8 == 0 && ((uintptr_t)x) % 16 == 0 && (C * esz) % 16 == 0 &&
-                    ((uintptr_t)codes) % 8 == 0 && cdiv(R, 128) <= 65535 && cdiv(C, 128) <= 0x7fffffff &&
-                    128 * C * 4 <= 0x7fffffffLL;
-  if (t_from_codes == 2 && !fast)
+  const bool fast = group == 128 && cdiv(R, 128) <= 65535 && 128 * C * 4 <= 0x7fffffffLL;
+  const bool vec = C % 8 == 0 && ((uintptr_t)x) % 16 == 0 && (C * esz) % 16 == 0 && ((uintptr_t)codes) % 8 == 0;
+  if (t_from_codes == 2 && !(fast && vec))
     return fail(KSD_EINVAL, "quantize_dual: the fp16 mode needs group 128, C %% 8 == 0 and 16-byte rows");
   if (!fast) {
     // the two single-layout kernels: row codes, then the transposed codes of x or of them
@@ -1115,8 +1156,12 @@ extern "C" int ksd_quantize_dual(const void *x, int x_dtype, int64_t R, int64_t 
   }
   const dim3 grid((unsigned)cdiv(C, 128), (unsigned)cdiv(R, 128));
 #define KSD_DUAL(DT)                                                                                      \
-  if (t_from_codes == 1)                                                                                  \
-    quant_dual_codes_kernel<DT><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t);         \
+  if (t_from_codes == 1 && vec)                                                                           \
+    quant_dual_codes_kernel<DT, true><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t);   \
+  else if (t_from_codes == 1)                                                                             \
+    quant_dual_codes_kernel<DT, false><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t);  \
+  else if (t_from_codes == 0 && !vec)                                                                     \
+    quant_dual_kernel<DT, false, false, false><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t); \
   else if (t_from_codes == 2)                                                                             \
     quant_dual_kernel<DT, false, true><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t);  \
   else                                                                                                    \
@@ -1140,11 +1185,12 @@ extern "C" int ksd_quantize_dual2(const void *x0, int64_t R0, int64_t C0, int8_t
   if (x_dtype != KSD_F32 && x_dtype != KSD_BF16 && x_dtype != KSD_F16)
     return fail(KSD_ETYPE, "quantize expects float32, bfloat16 or float16 input");
   const int esz = x_dtype == KSD_F32 ? 4 : 2;
-  auto fast = [&](const void *x, int64_t R, int64_t C, const int8_t *codes) {
-    return R > 0 && C > 0 && C % 8 == 0 && ((uintptr_t)x) % 16 == 0 && (C * esz) % 16 == 0 &&
-           ((uintptr_t)codes) % 8 == 0 && 128 * C * 4 <= 0x7fffffffLL;
+  auto fast = [&](int64_t R, int64_t C) { return R > 0 && C > 0 && 128 * C * 4 <= 0x7fffffffLL; };
+  auto vec16 = [&](const void *x, int64_t C, const int8_t *codes) {
+    return C % 8 == 0 && ((uintptr_t)x) % 16 == 0 && (C * esz) % 16 == 0 && ((uintptr_t)codes) % 8 == 0;
   };
-  if (!fast(x0, R0, C0, codes0) || !fast(x1, R1, C1, codes1) ||
+  const bool vec = vec16(x0, C0, codes0) && vec16(x1, C1, codes1);
+  if (!fast(R0, C0) || !fast(R1, C1) ||
       cdiv(C0, 128) * cdiv(R0, 128) + cdiv(C1, 128) * cdiv(R1, 128) > 0x7fffffffLL) {
     int rc = ksd_quantize_dual(x0, x_dtype, R0, C0, group, 1, codes0, scales0, codes_t0, scales_t0, stream);
     if (rc) return rc;
@@ -1156,11 +1202,15 @@ extern "C" int ksd_quantize_dual2(const void *x0, int64_t R0, int64_t C0, int8_t
   const DualOperand b{x1, R1, C1, codes1, scales1, codes_t1, scales_t1};
   const unsigned nblk = (unsigned)(cdiv(C0, 128) * cdiv(R0, 128) + cdiv(C1, 128) * cdiv(R1, 128));
   hipStream_t st = (hipStream_t)stream;
+#define KSD_DUAL2(DT)                                                             \
+  if (vec) quant_dual_codes2_kernel<DT, true><<<nblk, 512, 0, st>>>(a, b);        \
+  else quant_dual_codes2_kernel<DT, false><<<nblk, 512, 0, st>>>(a, b);
   switch (x_dtype) {
-    case KSD_F32: quant_dual_codes2_kernel<KSD_F32><<<nblk, 512, 0, st>>>(a, b); break;
-    case KSD_BF16: quant_dual_codes2_kernel<KSD_BF16><<<nblk, 512, 0, st>>>(a, b); break;
-    default: quant_dual_codes2_kernel<KSD_F16><<<nblk, 512, 0, st>>>(a, b); break;
+    case KSD_F32: KSD_DUAL2(KSD_F32); break;
+    case KSD_BF16: KSD_DUAL2(KSD_BF16); break;
+    default: KSD_DUAL2(KSD_F16); break;
   }
+#undef KSD_DUAL2
   return check_launch("quantize_dual2");
 }
 
@@ -1176,21 +1226,28 @@ extern "C" int ksd_quantize_dual_colsum(const void *x, int x_dtype, int64_t R, i
   if (!x || !codes || !scales || !codes_t || !scales_t || !colsum)
     return fail(KSD_EINVAL, "quantize_dual_colsum: null pointer");
   const int esz = x_dtype == KSD_F32 ? 4 : 2;
-  const bool fast = C % 8 == 0 && ((uintptr_t)x) % 16 == 0 && (C * esz) % 16 == 0 &&
-                    ((uintptr_t)codes) % 8 == 0 && cdiv(R, 128) <= 65535 && cdiv(C, 128) <= 0x7fffffff &&
-                    128 * C * 4 <= 0x7fffffffLL;
-  if (!fast) return fail(KSD_EINVAL, "quantize_dual_colsum: needs C %% 8 == 0 and 16-byte aligned rows");
+  if (cdiv(R, 128) > 65535 || 128 * C * 4 > 0x7fffffffLL)
+    return fail(KSD_EINVAL, "quantize_dual_colsum: tensor too large");
+  const bool vec = C % 8 == 0 && ((uintptr_t)x) % 16 == 0 && (C * esz) % 16 == 0 && ((uintptr_t)codes) % 8 == 0;
   const int64_t nt = cdiv(R, 128);
   if (!workspace || workspace_bytes < nt * C * 4 || ((uintptr_t)workspace) % 4 != 0)
     return fail(KSD_EINVAL, "quantize_dual_colsum: needs an fp32 workspace of %lld bytes",
                 (long long)(nt * C * 4));
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)cdiv(C, 128), (unsigned)nt);
+#define KSD_DUAL_SUM(DT)                                                                             \
+  if (vec)                                                                                           \
+    quant_dual_kernel<DT><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t, CeSrc{},  \
+                                                workspace);                                          \
+  else                                                                                               \
+    quant_dual_kernel<DT, false, false, false><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, \
+                                                                     scales_t, CeSrc{}, workspace);
   switch (x_dtype) {
-    case KSD_F32: quant_dual_kernel<KSD_F32><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t, CeSrc{}, workspace); break;
-    case KSD_BF16: quant_dual_kernel<KSD_BF16><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t, CeSrc{}, workspace); break;
-    default: quant_dual_kernel<KSD_F16><<<grid, 512, 0, st>>>(x, R, C, codes, scales, codes_t, scales_t, CeSrc{}, workspace); break;
+    case KSD_F32: KSD_DUAL_SUM(KSD_F32); break;
+    case KSD_BF16: KSD_DUAL_SUM(KSD_BF16); break;
+    default: KSD_DUAL_SUM(KSD_F16); break;
   }
+#undef KSD_DUAL_SUM
   hipLaunchKernelGGL(colsum_finalize_kernel, dim3((unsigned)cdiv(C, 256)), dim3(256), 0, st, workspace, nt, C, colsum);
   return check_launch("quantize_dual_colsum");
 }
@@ -1229,16 +1286,18 @@ extern "C" int ksd_ce_backward_quant_dual(const float *logits, int64_t R, int64_
     return fail(KSD_EINVAL, "ce_backward_quant_dual: null pointer");
   hipStream_t st = (hipStream_t)stream;
   const CeSrc ce{row_max, row_inv_sum, targets, ignore_index, grad_scale, dy_out};
-  const bool fast = C % 8 == 0 && ((uintptr_t)logits) % 16 == 0 && ((uintptr_t)codes) % 8 == 0 &&
-                    (dy_out == nullptr || ((uintptr_t)dy_out) % 16 == 0) && cdiv(R, 128) <= 65535 &&
-                    cdiv(C, 128) <= 0x7fffffff && 128 * C * 4 <= 0x7fffffffLL;
-  if (fast) {
+  if (cdiv(R, 128) <= 65535 && 128 * C * 4 <= 0x7fffffffLL) {
+    const bool vec = C % 8 == 0 && ((uintptr_t)logits) % 16 == 0 && ((uintptr_t)codes) % 8 == 0 &&
+                     (dy_out == nullptr || ((uintptr_t)dy_out) % 16 == 0);
     const dim3 grid((unsigned)cdiv(C, 128), (unsigned)cdiv(R, 128));
-    quant_dual_kernel<KSD_F32, true><<<grid, 512, 0, st>>>(logits, R, C, codes, scales, codes_t,
-                                                                  scales_t, ce);
+    if (vec)
+      quant_dual_kernel<KSD_F32, true><<<grid, 512, 0, st>>>(logits, R, C, codes, scales, codes_t, scales_t, ce);
+    else
+      quant_dual_kernel<KSD_F32, true, false, false><<<grid, 512, 0, st>>>(logits, R, C, codes, scales, codes_t,
+                                                                           scales_t, ce);
     return check_launch("ce_backward_quant_dual");
   }
-  // other shapes: dY into dy_out (required here), then the dual quantizer on it
+  // tensors past the tile kernel's 32-bit offsets: dY into dy_out (required here), then the dual quantizer on it
   if (!dy_out) return fail(KSD_EINVAL, "ce_backward_quant_dual: this shape needs dy_out (R x C fp32)");
   if (cdiv(R * C, 256) > 0x7fffffffLL) return fail(KSD_EINVAL, "ce_backward_quant_dual: tensor too large");
   ce_dy_kernel<<<(unsigned)cdiv(R * C, 256), 256, 0, st>>>(logits, R, C, ce);

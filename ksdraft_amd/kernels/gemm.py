@@ -11,6 +11,8 @@ linear layer and the KS3 cell.
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 import torch.nn.functional as F
 
@@ -49,26 +51,52 @@ def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t
 
 
-def _prepare(a_codes, a_scales, w_codes, w_scales, group):
+class _PadOperand(ctypes.Structure):  # KsdPadOperand of the C ABI
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("rows", ctypes.c_int64),
+                ("K", ctypes.c_int64), ("Kp", ctypes.c_int64)]
+
+
+def _pad_operands(dev, codes, K128):
+    """Each (rows, K) of ``codes`` zero-padded to its K of ``K128`` (None: left as it is), as
+    gemm.py:71-73 pads them: one launch for up to four operands, one buffer for their copies."""
+    codes = [t if k is None else t.contiguous() for t, k in zip(codes, K128)]
+    todo = [i for i, k in enumerate(K128) if k is not None]
+    buf = torch.empty(sum(codes[i].shape[0] * K128[i] for i in todo), dtype=torch.int8, device=dev)
+    args = (_PadOperand * len(todo))()
+    out, at = list(codes), 0
+    for n, i in enumerate(todo):
+        rows, K = codes[i].shape
+        out[i] = buf[at:at + rows * K128[i]].view(rows, K128[i])
+        args[n] = _PadOperand(codes[i].data_ptr(), out[i].data_ptr(), rows, K, K128[i])
+        at += rows * K128[i]
+    _lib.call("ksd_pad_codes", args, len(todo), _lib.stream_ptr(dev))
+    return out
+
+
+def _check_operands(a_codes, a_scales, w_codes, w_scales, group):
+    """Validation, the padded K (the kernel steps K by 128) and the padded scales. Codes are
+    zero-padded (gemm.py:71-73) by _pad_operands; groups smaller than 128 also pad the scale
+    columns of the padding groups (their codes are zero, so any finite scale leaves the sum
+    unchanged)."""
     M, N, K, n_groups, Kp = _validate(a_codes, a_scales, w_codes, w_scales, group)
     dev = _lib.require_gpu(a_codes, a_scales, w_codes, w_scales)
     if a_codes.dtype != torch.int8 or w_codes.dtype != torch.int8:
         raise TypeError("w8a8_gemm expects int8 codes")
     if a_scales.dtype != SCALE_DTYPE or w_scales.dtype != SCALE_DTYPE:
         raise TypeError("w8a8_gemm expects float16 scales")
-    # The kernel steps K by 128. Zero-pad codes (gemm.py:71-73) and, for groups smaller
-    # than 128, the scale columns of the padding groups (their codes are zero, so any
-    # finite scale leaves the sum unchanged).
     K128 = -(-Kp // 128) * 128
-    if K128 != K:
-        a_codes = F.pad(a_codes, (0, K128 - K))
-        w_codes = F.pad(w_codes, (0, K128 - K))
     g128 = K128 // group
     if g128 != n_groups:
         a_scales = F.pad(a_scales, (0, g128 - n_groups))
         w_scales = F.pad(w_scales, (0, g128 - n_groups))
-    return (dev, M, N, K128, _aligned(a_codes), a_scales.contiguous(), _aligned(w_codes),
-            w_scales.contiguous())
+    return dev, M, N, K128, a_scales.contiguous(), w_scales.contiguous()
+
+
+def _prepare(a_codes, a_scales, w_codes, w_scales, group):
+    dev, M, N, K128, a_scales, w_scales = _check_operands(a_codes, a_scales, w_codes, w_scales, group)
+    if K128 != a_codes.shape[1]:
+        a_codes, w_codes = _pad_operands(dev, (a_codes, w_codes), (K128, K128))
+    return dev, M, N, K128, _aligned(a_codes), a_scales, _aligned(w_codes), w_scales
 
 
 def w8a8_gemm_out(a_codes: torch.Tensor, a_scales: torch.Tensor, w_codes: torch.Tensor,
@@ -131,17 +159,23 @@ def w8a8_gemm_pair(first: tuple, second: tuple, group: int = GROUP_SIZE) -> tupl
     groups run the two GEMMs one after the other."""
     probs = []
     for a_codes, a_scales, w_codes, w_scales, out_dtype in (first, second):
-        dev, M, N, K, a, as_, w, ws = _prepare(a_codes, a_scales, w_codes, w_scales, group)
+        dev, M, N, K, as_, ws = _check_operands(a_codes, a_scales, w_codes, w_scales, group)
         code = _OUT_CODE.get(out_dtype)
         if code is None:
             raise TypeError(f"unsupported output dtype {out_dtype}")
-        probs.append((dev, M, N, K, a, as_, w, ws, code, out_dtype))
+        probs.append([dev, M, N, K, a_codes, as_, w_codes, ws, code, out_dtype])
     if group != GROUP_SIZE or any(p[3] == 0 for p in probs):
         return tuple(w8a8_gemm_out(a_codes, a_scales, w_codes, w_scales, group, out_dtype=dt)
                      for a_codes, a_scales, w_codes, w_scales, dt in (first, second))
     dev = probs[0][0]
     if probs[1][0] != dev:
         raise ValueError("w8a8_gemm_pair: both GEMMs must be on one device")
+    codes = [p[i] for p in probs for i in (4, 6)]
+    need = [p[3] if p[3] != t.shape[1] else None for p, t in zip((probs[0], probs[0], probs[1], probs[1]), codes)]
+    if any(k is not None for k in need):
+        codes = _pad_operands(dev, codes, need)
+    for n, p in enumerate(probs):
+        p[4], p[6] = _aligned(codes[2 * n]), _aligned(codes[2 * n + 1])
     outs = [torch.empty((M, N), dtype=dt, device=dev) for _, M, N, _, _, _, _, _, _, dt in probs]
     need = sum(gemm_splits(M, N, K) * M * N for _, M, N, K, *_ in probs
                if gemm_splits(M, N, K) > 1)
@@ -163,7 +197,6 @@ def gemm_splits(M: int, N: int, K: int, group: int = GROUP_SIZE) -> int:
     key = (M, N, K, group)
     s = _SPLITS.get(key)
     if s is None:
-        import ctypes
         c = ctypes.c_int(0)
         _lib.call("ksd_w8a8_gemm_splits", M, N, K, group, ctypes.byref(c))
         s = _SPLITS[key] = c.value

@@ -20,6 +20,8 @@ GROUP_SIZE = 128
 SCALE_DTYPE = torch.float16
 SCALE_MIN = 2.0 ** -24
 SCALE_MAX = 65504.0
+# widest rows of the dual quantizers' tile kernels (32-bit offsets within 128 fp32 rows)
+_DUAL_MAX_COLS = 0x7fffffff // 512
 
 
 def _padded_length(n: int, group: int = GROUP_SIZE) -> int:
@@ -202,15 +204,14 @@ def quantize_dual_colsum(g: torch.Tensor, group: int = GROUP_SIZE):
     gradient) from the same read of g: (codes, scales, codes_t, scales_t, colsum). The
     column sums run in another order than torch's sum (fp32, within rounding). Falls back to
     quantize_dual + torch's sum where the fused kernel does not apply (group other than 128,
-    C % 8 != 0, no rows)."""
+    no rows, tensors past its 32-bit tile offsets)."""
     g = _float_input(g)
     dev = _lib.require_gpu(g)
     if g.dim() != 2:
         raise ValueError("quantize_dual_colsum expects a 2-D tensor")
     g = g.contiguous()
     R, C = g.shape
-    esz = g.element_size()
-    if group != GROUP_SIZE or C % 8 or R == 0 or C == 0 or g.data_ptr() % 16 or (C * esz) % 16:
+    if group != GROUP_SIZE or R == 0 or C == 0 or R > 65535 * 128 or C > _DUAL_MAX_COLS:
         return (*quantize_dual(g, group), g.float().sum(0))
     codes = torch.empty((R, C), dtype=torch.int8, device=dev)
     scales = torch.empty((R, -(-C // group)), dtype=SCALE_DTYPE, device=dev)

@@ -14,7 +14,8 @@ import torch
 from .. import _lib
 from ..kernels.gemm import w8a8_gemm, w8a8_gemm_out, w8a8_gemm_pair
 from ..kernels.linear import w8a8_linear_forward_train
-from ..kernels.quant import GROUP_SIZE, SCALE_DTYPE, requant_transpose, requant_transpose_multi
+from ..kernels.quant import (_DUAL_MAX_COLS, GROUP_SIZE, SCALE_DTYPE, requant_transpose,
+                             requant_transpose_multi)
 
 IGNORE_INDEX = -100  # torch.nn.functional.cross_entropy's default
 
@@ -82,8 +83,9 @@ def cross_entropy_grad_int8(logits: torch.Tensor, targets: torch.Tensor, row_max
     scales = torch.empty((R, -(-C // group)), dtype=SCALE_DTYPE, device=dev)
     codes_t = torch.empty((C, R), dtype=torch.int8, device=dev)
     scales_t = torch.empty((C, -(-R // group)), dtype=SCALE_DTYPE, device=dev)
-    # shapes off the fused path (C % 8 != 0) stage dY in an fp32 buffer
-    dy = torch.empty((R, C), dtype=torch.float32, device=dev) if (return_dy or C % 8) else None
+    # tensors past the fused kernel's 32-bit tile offsets stage dY in an fp32 buffer
+    stage = R > 65535 * 128 or C > _DUAL_MAX_COLS
+    dy = torch.empty((R, C), dtype=torch.float32, device=dev) if (return_dy or stage) else None
     _lib.call("ksd_ce_backward_quant_dual", logits.data_ptr(), R, C, row_max.data_ptr(),
               row_inv_sum.data_ptr(), targets.data_ptr(), int(ignore_index), gsc.data_ptr(),
               group, codes.data_ptr(), scales.data_ptr(), codes_t.data_ptr(), scales_t.data_ptr(),
