@@ -176,11 +176,10 @@ __device__ __forceinline__ uint32_t lane_group_max(uint32_t v) {
 
 // Spine kernels: block = 512 threads = 16 rows x 32 lanes; a lane owns 4 consecutive
 // charts of the block's 128-chart segment (blockIdx.x), so a G-chart group is G/4 lanes of
-// one half-wave. Rows [blockIdx.y * kSpineRows, +kSpineRows), 2 per lane per iteration
+// one half-wave. Rows [blockIdx.y * rpb, +rpb), rpb a multiple of 64, 2 per lane per iteration
 // with both rows' loads issued first. The segment's increment table (128 charts x 256
 // indices) is staged in LDS with a pitch of 129 words (fp16 table) / 257 words (fp32):
 // lanes reading the same index of different charts then fall in different banks.
-constexpr int kSpineRows = 512;
 constexpr int kSpineThreads = 512;
 
 template <bool FUSED>
@@ -231,6 +230,33 @@ __device__ __forceinline__ float scale_of_finite(float h) {
   return f16_round(__builtin_elementwise_minimum(__builtin_elementwise_maximum(q, kScaleMin), kScaleMax));
 }
 
+// The composed contract's features of N coordinates x and their increments (ks3_int8.py:226-234).
+template <int N>
+__device__ __forceinline__ void composed_features(const float *x, const float *inc, float *f) {
+  float v[N], pre[N], q[N];
+  float near = 1.0f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    // relu (NaN-propagating max; -0 becomes +0, which leaves every output unchanged)
+    const float t = __builtin_elementwise_maximum(x[i] + inc[i], 0.0f);
+    v[i] = t;
+    pre[i] = scale_of_finite(t);  // amax over the rank dim (one element), :230-231
+    const float p = t * __builtin_amdgcn_rcpf(pre[i]);
+    q[i] = rintf(p);
+    near = fminf(near, fabsf(fabsf(p - q[i]) - 0.5f));
+  }
+  if (near < 0x1p-14f) {  // some quotient within 2^-14 of a half-integer: divide
+#pragma unroll
+    for (int i = 0; i < N; ++i) q[i] = rintf(v[i] / pre[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    // q = clamp(rint(h / pre), 0, 127); a NaN q leaves the feature NaN via pre
+    const float c = __builtin_amdgcn_fmed3f(q[i], 0.0f, 127.0f);
+    f[i] = f16_round(c * c) * (pre[i] * pre[i]);
+  }
+}
+
 // Composed contract (ks3_int8.py:205-234 + quantize_last_dim(h, G)): x is the fp16
 // coordinate; h = relu(x + inc[ti]); the rank-1 ReLU^2 requantization pre = fp16 scale of
 // |h|, code q = rint(h / pre) in [0, 127], feature fp16(q * q) * pre^2; then the feature's
@@ -241,7 +267,7 @@ __device__ __forceinline__ float scale_of_finite(float h) {
 template <int G, bool VEC>
 __global__ void __launch_bounds__(kSpineThreads) ks3_spine_kernel(
     const uint16_t *__restrict__ coords, int64_t M, int64_t F, const void *__restrict__ table,
-    float *__restrict__ h_out, int8_t *__restrict__ hq, uint16_t *__restrict__ hs, int64_t n_groups) {
+    float *__restrict__ h_out, int8_t *__restrict__ hq, uint16_t *__restrict__ hs, int64_t n_groups, int rpb) {
   using Tab = SpineTab<false>;
   __shared__ uint32_t tab[128 * Tab::kPitch];
   const int64_t c0 = (int64_t)blockIdx.x * 128;
@@ -254,8 +280,8 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_kernel(
   const bool seg_full = c0 + 128 <= F;             // block-uniform: no chart past F
   const int64_t colc = cok ? col0 : 0;             // a valid column for every lane
   const uint32_t tab_lane = (uint32_t)(uintptr_t)(tab) + (uint32_t)(lane * 4) * (4 * Tab::kPitch);
-  const int64_t row_end = min(M, (int64_t)(blockIdx.y + 1) * kSpineRows);
-  const int64_t rbase = (int64_t)blockIdx.y * kSpineRows, nrows = row_end - rbase;
+  const int64_t row_end = min(M, (int64_t)(blockIdx.y + 1) * rpb);
+  const int64_t rbase = (int64_t)blockIdx.y * rpb, nrows = row_end - rbase;
   const int64_t rfirst = rbase + rsub;
   // the two rows (r0, r0 + 16) of an iteration as packed fp16 words: 4 charts each
   auto raw2 = [&](int64_t r0, uint2 (&w)[2]) __attribute__((always_inline)) {
@@ -291,36 +317,12 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_kernel(
         typedef __attribute__((address_space(3))) const uint16_t lds_u16;
         inc[u][j] = f16_to_f32(*(lds_u16 *)(uintptr_t)(tab_lane + j * (4 * Tab::kPitch) + off[u][j]));
       }
-    float v[2][4], pre[2][4], h[2][4];
-    float near = 1.0f;
+    float h[2][4];
+    composed_features<8>(&x[0][0], &inc[0][0], &h[0][0]);
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        // relu (NaN-propagating max; -0 becomes +0, which leaves every output unchanged)
-        const float t = __builtin_elementwise_maximum(x[u][j] + inc[u][j], 0.0f);
-        v[u][j] = t;
-        pre[u][j] = scale_of_finite(t);  // amax over the rank dim (one element), :230-231
-        const float p = t * __builtin_amdgcn_rcpf(pre[u][j]);
-        const float r = rintf(p);
-        near = fminf(near, fabsf(fabsf(p - r) - 0.5f));
-        h[u][j] = r;
-      }
-    if (near < 0x1p-14f) {  // some quotient within 2^-14 of a half-integer: divide
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) h[u][j] = rintf(v[u][j] / pre[u][j]);
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        // q = clamp(rint(h / pre), 0, 127); a NaN q leaves the feature NaN via pre
-        const float q = __builtin_amdgcn_fmed3f(h[u][j], 0.0f, 127.0f);
-        const float f = f16_round(q * q) * (pre[u][j] * pre[u][j]);
-        h[u][j] = seg_full || (VEC ? cok : col0 + j < F) ? f : 0.0f;
-      }
+      for (int j = 0; j < 4; ++j) h[u][j] = seg_full || (VEC ? cok : col0 + j < F) ? h[u][j] : 0.0f;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int64_t row = r0 + 16 * u;
@@ -365,7 +367,7 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_kernel(
   raw2(rfirst, wa);
   raw2(rfirst + 32, wb);
 #pragma unroll 1
-  for (int it = 0; it < kSpineRows / 64; ++it) {
+  for (int it = 0; it < rpb / 64; ++it) {
     const int64_t r0 = rfirst + 64 * it;
     const uint2 ca[2] = {wa[0], wa[1]};
     raw2(r0 + 64, wa);
@@ -374,6 +376,37 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_kernel(
     raw2(r0 + 96, wb);
     body(r0 + 32, cb);
   }
+}
+
+// The fused contract behind the coordinate (ks3_triton.py:72-75, 150-156) for a lane's 4 charts
+// of a row, one G-chart group being G/4 adjacent lanes: the group's pre-scale, the ReLU^2 codes
+// and features, their scale s and packed codes.
+template <int G>
+__device__ __forceinline__ void fused_requant(const float (&h)[4], float &s, uint32_t &wq) {
+  const uint32_t am = lane_group_max<G / 4>(__builtin_bit_cast(uint32_t, abs_max<4>(h)));
+  const float pre = group_scale(__builtin_bit_cast(float, am));
+  const float rp = __builtin_amdgcn_rcpf(pre);
+  float t[4];
+  float near = 1.0f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float p = h[j] * rp;
+    t[j] = rintf(p);
+    near = fminf(near, fabsf(fabsf(p - t[j]) - 0.5f));
+  }
+  if (near < 0x1p-14f) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) t[j] = rintf(h[j] / pre);
+  }
+  float f[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float q = __builtin_amdgcn_fmed3f(t[j], 0.0f, 127.0f);  // NaN q: NaN via pre
+    f[j] = (q * q) * (pre * pre);
+  }
+  const uint32_t hm = lane_group_max<G / 4>(__builtin_bit_cast(uint32_t, abs_max<4>(f)));
+  s = group_scale(__builtin_bit_cast(float, hm));
+  codes_rcp_packed<4>(f, s, &wq);
 }
 
 // The fused-kernel contract of project_fused / _fused_gemm_spine, 'int8' mode
@@ -386,7 +419,7 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_kernel(
 template <int G, bool VEC>
 __global__ void __launch_bounds__(kSpineThreads) ks3_spine_fused_kernel(
     const float *__restrict__ acc, int64_t M, int64_t F, const void *__restrict__ table,
-    int8_t *__restrict__ hq, uint16_t *__restrict__ hs, int64_t n_groups) {
+    int8_t *__restrict__ hq, uint16_t *__restrict__ hs, int64_t n_groups, int rpb) {
   using Tab = SpineTab<true>;
   __shared__ uint32_t tab[128 * Tab::kPitch];
   const int64_t c0 = (int64_t)blockIdx.x * 128;
@@ -399,8 +432,8 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_fused_kernel(
   const bool seg_full = c0 + 128 <= F;
   const int64_t colc = cok ? col0 : 0;
   const uint32_t tab_lane = (uint32_t)(uintptr_t)(tab) + (uint32_t)(lane * 4) * (4 * Tab::kPitch);
-  const int64_t row_end = min(M, (int64_t)(blockIdx.y + 1) * kSpineRows);
-  const int64_t rbase = (int64_t)blockIdx.y * kSpineRows, nrows = row_end - rbase;
+  const int64_t row_end = min(M, (int64_t)(blockIdx.y + 1) * rpb);
+  const int64_t rbase = (int64_t)blockIdx.y * rpb, nrows = row_end - rbase;
   const int64_t rfirst = rbase + rsub;
   auto raw2 = [&](int64_t r0, float4 (&w)[2]) __attribute__((always_inline)) {
 #pragma unroll
@@ -440,31 +473,9 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_fused_kernel(
     for (int u = 0; u < 2; ++u) {
       const int64_t row = r0 + 16 * u;
       const bool rok = row < row_end;
-      const uint32_t am = lane_group_max<G / 4>(__builtin_bit_cast(uint32_t, abs_max<4>(h[u])));
-      const float pre = group_scale(__builtin_bit_cast(float, am));
-      const float rp = __builtin_amdgcn_rcpf(pre);
-      float t[4];
-      float near = 1.0f;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float p = h[u][j] * rp;
-        t[j] = rintf(p);
-        near = fminf(near, fabsf(fabsf(p - t[j]) - 0.5f));
-      }
-      if (near < 0x1p-14f) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) t[j] = rintf(h[u][j] / pre);
-      }
-      float f[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float q = __builtin_amdgcn_fmed3f(t[j], 0.0f, 127.0f);  // NaN q: NaN via pre
-        f[j] = (q * q) * (pre * pre);
-      }
-      const uint32_t hm = lane_group_max<G / 4>(__builtin_bit_cast(uint32_t, abs_max<4>(f)));
-      const float s = group_scale(__builtin_bit_cast(float, hm));
+      float s;
       uint32_t wq;
-      codes_rcp_packed<4>(f, s, &wq);
+      fused_requant<G>(h[u], s, wq);
       const int64_t lr = row - rbase;  // block-uniform descriptors, as in ks3_spine_kernel
       const bool lead = rok && cok && (lane & (G / 4 - 1)) == 0;
       __builtin_amdgcn_raw_buffer_store_b16(scale_bits(s), rsrc(hs + rbase * n_groups, 2 * nrows * n_groups),
@@ -483,7 +494,7 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_fused_kernel(
   raw2(rfirst, wa);
   raw2(rfirst + 32, wb);
 #pragma unroll 1
-  for (int it = 0; it < kSpineRows / 64; ++it) {
+  for (int it = 0; it < rpb / 64; ++it) {
     const int64_t r0 = rfirst + 64 * it;
     const float4 ca[2] = {wa[0], wa[1]};
     raw2(r0 + 64, wa);
@@ -491,6 +502,87 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_fused_kernel(
     const float4 cb[2] = {wb[0], wb[1]};
     raw2(r0 + 96, wb);
     body(r0 + 32, cb);
+  }
+}
+
+// Either spine on few rows (M F up to kDirectValues): the same values without the table, whose kernel
+// evaluates 256 indices of every chart and whose readers first copy 64 or 128 KB of it into LDS. Block =
+// 8 rows x 32 lanes of a 128-chart segment; a lane evaluates its row's 4 increments itself, about 80
+// VALU instructions each (six divisions by 127), so its time grows with M F where the table's reader
+// takes 30 us at least. Measured (us, the fused contract, table and reader -> this kernel): 16 x 5888
+// 39.8 -> 3.8, 256 x 5888 37.4 -> 8.8, 1024 x 5888 36.1 -> 26.2, 3001 x 256 30.6 -> 5.8.
+template <bool FUSED, int G, bool VEC>
+__global__ void __launch_bounds__(256) ks3_spine_rows_kernel(
+    const void *__restrict__ in, int64_t M, int64_t F, const int8_t *__restrict__ spine_codes,
+    const uint16_t *__restrict__ spine_scale, const uint16_t *__restrict__ sc16,
+    const uint16_t *__restrict__ sh16, const int8_t *__restrict__ tanh_lut, float *__restrict__ h_out,
+    int8_t *__restrict__ hq, uint16_t *__restrict__ hs, int64_t n_groups) {
+  __shared__ int8_t lut[256];
+  if (threadIdx.x < 64) ((uint32_t *)lut)[threadIdx.x] = ((const uint32_t *)tanh_lut)[threadIdx.x];
+  const int lane = threadIdx.x & 31;
+  const int64_t row = (int64_t)blockIdx.y * 8 + (threadIdx.x >> 5);
+  const int64_t col0 = (int64_t)blockIdx.x * 128 + lane * 4, at = min(row, M - 1) * F + col0;
+  float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (VEC && col0 < F) {
+    if constexpr (FUSED) {
+      const float4 v = *(const float4 *)((const float *)in + at);
+      x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+    } else {
+      const uint2 v = *(const uint2 *)((const uint16_t *)in + at);
+      x[0] = f16_to_f32((uint16_t)v.x);
+      x[1] = f16_to_f32((uint16_t)(v.x >> 16));
+      x[2] = f16_to_f32((uint16_t)v.y);
+      x[3] = f16_to_f32((uint16_t)(v.y >> 16));
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (col0 + j < F) x[j] = FUSED ? ((const float *)in)[at + j] : f16_to_f32(((const uint16_t *)in)[at + j]);
+  }
+  __syncthreads();
+  float h[4], inc[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const bool ok = col0 + j < F;
+    const SpineCol c = load_spine_col(spine_codes, spine_scale, sc16, sh16, col0 + j, ok);
+    if constexpr (FUSED) {
+      const float xc = fminf(fmaxf(x[j], -kScaleMax), kScaleMax);  // a NaN -> -65504
+      const int ti = min(max(lut_index_f32(xc * 0.25f), -128), 127);
+      h[j] = ok ? xc + (float)spine_sum<true>(ti, c, lut) * (c.ps / 64.0f) : 0.0f;
+    } else {
+      const int td = spine_sum<false>(lut_index_x(x[j]), c, lut) / 64;  // rounding_mode="trunc"
+      inc[j] = f16_round(f16_round((float)td) * c.ps);
+    }
+  }
+  if constexpr (!FUSED) {
+    float f[4];
+    composed_features<4>(x, inc, f);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h[j] = col0 + j < F ? f[j] : 0.0f;
+  }
+  const bool rok = row < M;
+  if (!FUSED && h_out && rok) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (col0 + j < F) h_out[row * F + col0 + j] = h[j];
+  }
+  if (!FUSED && !hq) return;
+  float s;
+  uint32_t wq;
+  if constexpr (FUSED) {
+    fused_requant<G>(h, s, wq);
+  } else {  // quantize_last_dim(h, G)
+    s = group_scale(__builtin_bit_cast(float, lane_group_max<G / 4>(__builtin_bit_cast(uint32_t, abs_max<4>(h)))));
+    codes_rcp_packed<4>(h, s, &wq);
+  }
+  if (!rok || col0 >= F) return;
+  if ((lane & (G / 4 - 1)) == 0) hs[row * n_groups + col0 / G] = scale_bits(s);
+  if (VEC) {
+    *(uint32_t *)(hq + row * F + col0) = wq;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (col0 + j < F) hq[row * F + col0 + j] = (int8_t)(wq >> (8 * j));
   }
 }
 
@@ -966,24 +1058,73 @@ __global__ void ks3_tanh16_kernel(const uint16_t *__restrict__ x, int64_t n, uin
 // ---------------------------------------------------------------- launchers
 template <int G>
 static void launch_spine(bool vec, dim3 grid, hipStream_t st, const uint16_t *coords, int64_t M,
-                         int64_t F, const void *table, float *h, int8_t *hq, uint16_t *hs, int64_t ng) {
+                         int64_t F, const void *table, float *h, int8_t *hq, uint16_t *hs, int64_t ng, int rpb) {
   if (vec)
     hipLaunchKernelGGL((ks3_spine_kernel<G, true>), grid, dim3(kSpineThreads), 0, st, coords, M, F,
-                       table, h, hq, hs, ng);
+                       table, h, hq, hs, ng, rpb);
   else
     hipLaunchKernelGGL((ks3_spine_kernel<G, false>), grid, dim3(kSpineThreads), 0, st, coords, M, F,
-                       table, h, hq, hs, ng);
+                       table, h, hq, hs, ng, rpb);
 }
 
 template <int G>
 static void launch_fused(bool vec, dim3 grid, hipStream_t st, const float *acc, int64_t M,
-                         int64_t F, const void *table, int8_t *hq, uint16_t *hs, int64_t ng) {
+                         int64_t F, const void *table, int8_t *hq, uint16_t *hs, int64_t ng, int rpb) {
   if (vec)
     hipLaunchKernelGGL((ks3_spine_fused_kernel<G, true>), grid, dim3(kSpineThreads), 0, st, acc, M,
-                       F, table, hq, hs, ng);
+                       F, table, hq, hs, ng, rpb);
   else
     hipLaunchKernelGGL((ks3_spine_fused_kernel<G, false>), grid, dim3(kSpineThreads), 0, st, acc,
-                       M, F, table, hq, hs, ng);
+                       M, F, table, hq, hs, ng, rpb);
+}
+
+// Where the table-free kernel is the faster one: at 1024 x 5888 (6.0e6 values) 26.2 against 36.1 us, at
+// 3001 x 2944 (8.8e6) 37.3 against 33.9.
+constexpr int64_t kDirectValues = 7 << 20;
+static bool spine_direct(int64_t M, int64_t F) { return M <= 8 * 65535 && M <= kDirectValues / F; }
+
+template <bool FUSED, int G>
+static void launch_rows(bool vec, hipStream_t st, const void *in, int64_t M, int64_t F,
+                        const int8_t *spine_codes, const uint16_t *spine_scale, const uint16_t *sc16,
+                        const uint16_t *sh16, const int8_t *tanh_lut, float *h, int8_t *hq, uint16_t *hs) {
+  const dim3 grid((unsigned)cdiv(F, 128), (unsigned)cdiv(M, 8));
+  if (vec)
+    hipLaunchKernelGGL((ks3_spine_rows_kernel<FUSED, G, true>), grid, dim3(256), 0, st, in, M, F, spine_codes,
+                       spine_scale, sc16, sh16, tanh_lut, h, hq, hs, cdiv(F, G));
+  else
+    hipLaunchKernelGGL((ks3_spine_rows_kernel<FUSED, G, false>), grid, dim3(256), 0, st, in, M, F, spine_codes,
+                       spine_scale, sc16, sh16, tanh_lut, h, hq, hs, cdiv(F, G));
+}
+template <bool FUSED>
+static int launch_rows_g(int group, bool vec, hipStream_t st, const void *in, int64_t M, int64_t F,
+                         const int8_t *spine_codes, const uint16_t *spine_scale, const uint16_t *sc16,
+                         const uint16_t *sh16, const int8_t *tanh_lut, float *h, int8_t *hq, uint16_t *hs) {
+#define KSD_ROWS_ARGS vec, st, in, M, F, spine_codes, spine_scale, sc16, sh16, tanh_lut, h, hq, hs
+  switch (group) {
+    case 32: launch_rows<FUSED, 32>(KSD_ROWS_ARGS); break;
+    case 64: launch_rows<FUSED, 64>(KSD_ROWS_ARGS); break;
+    default: launch_rows<FUSED, 128>(KSD_ROWS_ARGS); break;
+  }
+#undef KSD_ROWS_ARGS
+  return check_launch("ks3_spine (rows)");
+}
+
+// Rows per block of a table reader. A CU's time goes with the rows it works through, each of its n blocks
+// adding the table's copy into LDS: n (rpb + stage), where the fused reader copies 128 KB and has a CU to
+// itself (6 us, some 128 rows) and the composed one's copy runs beside the other block of its CU (16), a
+// block alone on its CU losing about a tenth. Other than 512 rows only for a gain of a twentieth. Before
+// and after (us, 512 rows -> this): fused 3001 x 5888 61.8 -> 42.2, 8192 x 5888 91.0 -> 85.7, 8192 x 2944
+// 61.9 -> 46.2; composed 3001 x 5888 52.3 -> 37.8, 4096 x 5888 52.5 -> 43.4, 8192 x 1536 33.1 -> 25.8.
+static int spine_rows_per_block(bool fused, int64_t M, int64_t F) {
+  const int64_t segs = cdiv(F, 128), cus = cu_count();
+  auto cost = [&](int64_t rpb) {
+    const int64_t n = cdiv(segs * cdiv(M, rpb), cus);
+    return 20 * n * (rpb + (fused ? 128 : 16)) * (!fused && n == 1 ? 11 : 10);
+  };
+  int64_t best = 512, least = cost(512) / 20 * 19;
+  for (int64_t rpb = 64; rpb <= 1024 && rpb <= (1LL << 30) / F; rpb += 64)
+    if (cost(rpb) < least) best = rpb, least = cost(rpb);
+  return (int)best;
 }
 
 static int64_t vjp_row_blocks(int64_t M) { return cdiv(M, kVjpRowsPerBlock); }
@@ -1253,6 +1394,14 @@ using namespace ksd;
 
 // The fused contract's per-chart increment table (F x 256 fp32), for the fused projection
 // GEMM in gemm.hip.
+int ksd::ks3_fused_rows(const float *acc, int64_t M, int64_t F, const int8_t *spine_codes,
+                        const uint16_t *spine_scale, const uint16_t *warp_scale, const uint16_t *warp_shift,
+                        const int8_t *tanh_lut, int group, int8_t *h_codes, uint16_t *h_scales, hipStream_t st) {
+  const bool vec = (F & 3) == 0 && ((uintptr_t)acc & 15) == 0 && ((uintptr_t)h_codes & 3) == 0;
+  return launch_rows_g<true>(group, vec, st, acc, M, F, spine_codes, spine_scale, warp_scale, warp_shift,
+                             tanh_lut, nullptr, h_codes, h_scales);
+}
+
 int ksd::ks3_fused_table(const int8_t *spine_codes, const uint16_t *spine_scale,
                          const uint16_t *warp_scale, const uint16_t *warp_shift, const int8_t *tanh_lut,
                          int64_t F, float *table, hipStream_t st) {
@@ -1271,10 +1420,10 @@ static int spine_checks(const char *who, const void *in, int64_t M, int64_t F, c
     return fail(KSD_EINVAL, "%s: null input pointer", who);
   if (!table || ((uintptr_t)table & 15) != 0)
     return fail(KSD_EINVAL, "%s: table workspace must be a 16-byte aligned buffer", who);
-  // stores address a block's kSpineRows rows from one base with 32-bit offsets
-  if (F > (1LL << 31) / (2 * kSpineRows)) return fail(KSD_EINVAL, "%s: F too large", who);
+  // stores address a block's rows from one base with 32-bit offsets (spine_rows_per_block)
+  if (F > (1LL << 31) / 1024) return fail(KSD_EINVAL, "%s: F too large", who);
   if (((uintptr_t)tanh_lut & 3) != 0) return fail(KSD_EINVAL, "%s: tanh_lut must be 4-byte aligned", who);
-  if (cdiv(M, kSpineRows) > 0x7fffffff) return fail(KSD_EINVAL, "%s: M too large", who);
+  if (cdiv(M, 512) > 0x7fffffff) return fail(KSD_EINVAL, "%s: M too large", who);
   return KSD_OK;
 }
 
@@ -1293,11 +1442,15 @@ extern "C" int ksd_ks3_spine_fwd(const uint16_t *coords, int64_t M, int64_t F,
   const bool vec = (F & 3) == 0 && ((uintptr_t)coords & 7) == 0 && ((uintptr_t)h & 15) == 0 &&
                    ((uintptr_t)h_codes & 3) == 0;
   const int64_t ng = cdiv(F, group);
-  dim3 grid((unsigned)cdiv(F, 128), (unsigned)cdiv(M, kSpineRows));
   hipStream_t st = (hipStream_t)stream;
+  if (spine_direct(M, F))
+    return launch_rows_g<false>(group, vec, st, coords, M, F, spine_codes, spine_scale, warp_scale, warp_shift,
+                                tanh_lut, h, h_codes, h_scales);
+  const int rpb = spine_rows_per_block(false, M, F);
+  dim3 grid((unsigned)cdiv(F, 128), (unsigned)cdiv(M, rpb));
   hipLaunchKernelGGL(ks3_spine_table_kernel<false>, dim3((unsigned)F), dim3(256), 0, st, spine_codes,
                      spine_scale, warp_scale, warp_shift, tanh_lut, (void *)table);
-#define KSD_SPINE_ARGS vec, grid, st, coords, M, F, table, h, h_codes, h_scales, ng
+#define KSD_SPINE_ARGS vec, grid, st, coords, M, F, table, h, h_codes, h_scales, ng, rpb
   switch (group) {
     case 32: launch_spine<32>(KSD_SPINE_ARGS); break;
     case 64: launch_spine<64>(KSD_SPINE_ARGS); break;
@@ -1374,11 +1527,15 @@ extern "C" int ksd_ks3_spine_fused(const float *acc, int64_t M, int64_t F,
   if (M == 0 || F == 0) return KSD_OK;
   const bool vec = (F & 3) == 0 && ((uintptr_t)acc & 15) == 0 && ((uintptr_t)h_codes & 3) == 0;
   const int64_t ng = cdiv(F, group);
-  dim3 grid((unsigned)cdiv(F, 128), (unsigned)cdiv(M, kSpineRows));
   hipStream_t st = (hipStream_t)stream;
+  if (spine_direct(M, F))
+    return ks3_fused_rows(acc, M, F, spine_codes, spine_scale, warp_scale, warp_shift, tanh_lut, group,
+                          h_codes, h_scales, st);
+  const int rpb = spine_rows_per_block(true, M, F);
+  dim3 grid((unsigned)cdiv(F, 128), (unsigned)cdiv(M, rpb));
   hipLaunchKernelGGL(ks3_spine_table_kernel<true>, dim3((unsigned)F), dim3(256), 0, st, spine_codes,
                      spine_scale, warp_scale, warp_shift, tanh_lut, (void *)table);
-#define KSD_FUSED_ARGS vec, grid, st, acc, M, F, table, h_codes, h_scales, ng
+#define KSD_FUSED_ARGS vec, grid, st, acc, M, F, table, h_codes, h_scales, ng, rpb
   switch (group) {
     case 32: launch_fused<32>(KSD_FUSED_ARGS); break;
     case 64: launch_fused<64>(KSD_FUSED_ARGS); break;

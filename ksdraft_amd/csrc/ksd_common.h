@@ -54,10 +54,20 @@ static inline int cu_count() {
   return n;
 }
 
+// ks3.hip: the fused contract's spine on the accumulator (M, F) without a table.
+int ks3_fused_rows(const float *acc, int64_t M, int64_t F, const int8_t *spine_codes,
+                   const uint16_t *spine_scale, const uint16_t *warp_scale, const uint16_t *warp_shift,
+                   const int8_t *tanh_lut, int group, int8_t *h_codes, uint16_t *h_scales, hipStream_t st);
+
 // ks3.hip: launches the fused contract's per-chart increment table kernel (F x 256 fp32).
 int ks3_fused_table(const int8_t *spine_codes, const uint16_t *spine_scale, const uint16_t *warp_scale,
                     const uint16_t *warp_shift, const int8_t *tanh_lut, int64_t F, float *table,
                     hipStream_t st);
+
+// rows.hip: the group-128 GEMM for few rows, and the shapes it is the faster one for.
+bool rows_gemm_fits(int64_t M, int64_t N, int64_t K);
+void rows_gemm(const int8_t *a, const uint16_t *as, const int8_t *w, const uint16_t *ws, int M, int N, int K,
+               int splits, const float *bias, const void *residual, void *y, int out, hipStream_t st);
 
 // ---------------------------------------------------------------- device numerics
 constexpr float kScaleMin = 5.9604644775390625e-08f;  // 2**-24, quant.py:22

@@ -40,6 +40,7 @@ from .quant import (GROUP_SIZE, dequantize_last_dim, quantize_dual, quantize_las
 
 TANH_DOMAIN = 3.2
 FP16 = torch.float16
+_GEMM_OUT = (torch.float32, torch.bfloat16, torch.float16)
 
 
 def make_tanh_lut(device) -> torch.Tensor:
@@ -453,7 +454,7 @@ class KS3Int8Cell(nn.Module):
         the result is residual + cell(x), the add done in the up-projection's store."""
         out_dt = self._out_dtype(x)
         fuse = (residual is not None and residual.dtype == out_dt
-                and out_dt in (torch.float32, torch.bfloat16, torch.float16))
+                and out_dt in _GEMM_OUT)
         if self.trainable:
             y = _KS3Int8Train.apply(
                 x, self.master_down, self.master_up, self.master_coefficients,
@@ -461,7 +462,8 @@ class KS3Int8Cell(nn.Module):
             return y if fuse or residual is None else residual + y
         self._check_supported()
         x2 = x.reshape(-1, x.shape[-1])
-        xq, xs = quantize_last_dim(x2.float(), self.group)
+        # 16-bit input quantizes as its exact fp32 values would, without that copy
+        xq, xs = quantize_last_dim(x2 if x2.dtype in _GEMM_OUT else x2.float(), self.group)
         from .ks3_triton import project_fused
         scale_dq, shift_dq = self._warp_scalars(FP16)
         hq, hs = project_fused(
@@ -473,7 +475,8 @@ class KS3Int8Cell(nn.Module):
             y = w8a8_gemm_out(hq, hs, self.up_codes, self.up_scales, self.group, out_dtype=out_dt,
                               residual=residual.reshape(-1, self.out_features))
             return y.reshape(*x.shape[:-1], self.out_features)
-        y = w8a8_gemm(hq, hs, self.up_codes, self.up_scales, self.group)
+        y = w8a8_gemm_out(hq, hs, self.up_codes, self.up_scales, self.group,
+                          out_dtype=out_dt if out_dt in _GEMM_OUT else torch.float32)
         y = y.reshape(*x.shape[:-1], self.out_features).to(out_dt)
         return y if residual is None else residual + y
 
@@ -498,15 +501,16 @@ class _KS3Int8Train(torch.autograd.Function):
     @staticmethod
     def forward(ctx, inputs, down, up, coefficients, raw_scale, raw_shift, cell, residual=None):
         cell._repack_masters()
-        x = inputs.reshape(-1, inputs.shape[-1]).float()
-        xq, xs = quantize_last_dim(x, cell.group)
+        x = inputs.reshape(-1, inputs.shape[-1])
+        xq, xs = quantize_last_dim(x if x.dtype in _GEMM_OUT else x.float(), cell.group)
         hq, hs, coords16 = cell._project_codes(xq, xs)
         out_dt = cell._out_dtype(inputs)
         if residual is not None:  # residual + y, added in the up-projection's store
             y = w8a8_gemm_out(hq, hs, cell.up_codes, cell.up_scales, cell.group, out_dtype=out_dt,
                               residual=residual.reshape(-1, cell.out_features))
         else:
-            y = w8a8_gemm(hq, hs, cell.up_codes, cell.up_scales, cell.group)
+            y = w8a8_gemm_out(hq, hs, cell.up_codes, cell.up_scales, cell.group,
+                              out_dtype=out_dt if out_dt in _GEMM_OUT else torch.float32)
         ctx.cell = cell
         ctx.input_shape = inputs.shape
         ctx.has_residual = residual is not None

@@ -5,20 +5,18 @@ the per-group requantization (ks3_triton.py:100-156), following the fused kernel
 arithmetic contract, not the composed one.
 
 * 'int8' (NL == 2) with group 128, up to ONE_LAUNCH_MAX_ROWS rows (the eval path's
-  decode and short-prefill shapes): the reference's single-kernel form,
-  ksd_ks3_project_fused, a GEMM whose epilogue runs the fused contract (fp32 coordinates
-  and LUT index, no truncation, group pre-scale, second requantization) on each finished
-  fp32 accumulator tile and stores only the h codes and scales, after a small kernel has
-  tabulated the per-chart increments. Its accumulator is the unsplit ordered sum over all
-  K groups, so it is taken only where the standalone GEMM would not split K either: the
-  outputs are then identical to the two-launch form's. At d 1536, F 5888 on MI355X it
-  takes about 29 us against 49-53 us for M <= 256 and 53 against 58 us at M = 1024.
-* 'int8' otherwise: ksd_w8a8_gemm_nt (fp32 accumulator out), then ksd_ks3_spine_fused,
-  the same per-element arithmetic with the per-chart table staged in LDS per 128-chart
-  segment. At M >= 2048 this is the faster form (223 against 254 us at M 8192): in one
-  launch the table (128 KB per 128-chart tile) cannot sit in LDS beside the GEMM's
-  132 KB operand ring, so the epilogue gathers it from L2, and the spine's VALU work runs
-  between the MFMA steps instead of beside them. ``one_launch`` forces either form.
+  decode and short-prefill shapes): ksd_ks3_project_fused, one call that keeps the GEMM's
+  accumulator in its workspace and runs the fused contract on it (fp32 coordinates and LUT
+  index, no truncation, group pre-scale, second requantization). Its accumulator is the
+  unsplit ordered sum over all K groups, so it is taken only where the standalone GEMM would
+  not split K either: the outputs are then identical to the other form's. At d 1536, F 5888
+  on MI355X it takes 9 us at M = 16 and 22 at M = 256.
+* 'int8' otherwise: ksd_w8a8_gemm_nt (fp32 accumulator out), then ksd_ks3_spine_fused, the
+  same per-element arithmetic. ``one_launch=True`` forces ksd_ks3_project_fused, which past
+  256 rows is the reference's single-kernel form: a GEMM whose epilogue runs the contract on
+  each finished tile, with no accumulator in memory, and slower for it (36.4 against 27.5 us
+  at M 512): the per-chart table (128 KB per 128-chart tile) cannot sit in LDS beside the
+  GEMM's operand ring, so the epilogue gathers it from L2.
 * 'fp16' and 'fp32' (NL == 1, 0; ks3_triton.py:76-98): ksd_ks3_spine_float on the
   accumulator (the coordinates not rounded to fp16, the warp scalars in fp16), every
   fp16/fp32 op of the Triton source rounded separately.
@@ -47,8 +45,8 @@ def project_fused(
     """Input projection + Horner spine + requant (ks3_triton.py:159-195).
 
     warp_scale/warp_shift: dequantized fp16 per-chart scalars. one_launch: None picks the
-    form by shape (see above); True forces the single launch ('int8', group 128 only),
-    False the two launches. Returns (h_codes int8 (M, N), h_scales fp16 (M, ceil(N/group)))."""
+    form by shape (see above); True forces ksd_ks3_project_fused ('int8', group 128 only),
+    False the GEMM and the spine. Returns (h_codes int8 (M, N), h_scales fp16 (M, ceil(N/group)))."""
     if group & (group - 1):
         raise ValueError("group must be a power of two (32 or 128)")
     nl = {"fp32": 0, "fp16": 1, "int8": 2}[nonlinear]
@@ -70,10 +68,11 @@ def project_fused(
     return hq, hs
 
 
-# Largest M for which project_fused takes the single launch by default (measured on MI355X
-# at d 1536, F 5888: 29 against 49-53 us up to M 256, 53 against 58 us at M 1024, 75
-# against 69 us at M 2048).
-ONE_LAUNCH_MAX_ROWS = 1024
+# Largest M for which project_fused takes ksd_ks3_project_fused by default: up to it the entry
+# keeps the accumulator in its table workspace and takes the table-free spine; past it, the GEMM
+# with its own accumulator and ksd_ks3_spine_fused is faster than the single launch (M 512:
+# 27.5 against 36.4 us, M 1024: 52.5 against 62.4).
+ONE_LAUNCH_MAX_ROWS = 256
 
 
 def _one_launch_pays(a_codes: torch.Tensor, w_codes: torch.Tensor) -> bool:
@@ -89,7 +88,7 @@ def _one_launch_pays(a_codes: torch.Tensor, w_codes: torch.Tensor) -> bool:
 
 def _project_fused_int8(a_codes, a_scales, w_codes, w_scales, spine_codes, spine_scale,
                         warp_scale16, warp_shift16, tanh_lut):
-    """GEMM + spine + requantization in one launch (group 128, 'int8'); None for K = 0,
+    """GEMM + spine + requantization in one call (group 128, 'int8'); None for K = 0,
     which the two-launch path covers (its GEMM returns zeros)."""
     dev, M, N, K, a, as_, w, ws = _prepare(a_codes, a_scales, w_codes, w_scales, 128)
     if K == 0:
