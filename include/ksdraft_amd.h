@@ -60,6 +60,20 @@ int ksd_quantize_lastdim(const void *x, int x_dtype, int64_t rows, int64_t K,
                          const float *noise, float dither2, void *stream);
 
 /*
+ * The eval forward of an int8 linear layer (reference ksdraft/kernels/linear.py:62-73): quantizes
+ * the fp32 master w (N, K) and the tokens x (M, K) along K in one launch (two where a row is not
+ * 16-byte aligned), then ksd_w8a8_gemm_nt_ex on the codes. The same outputs as the three calls.
+ *   K            a positive multiple of 128 (group 128)
+ *   x            of type x_dtype, row stride x_stride elements; w dense
+ *   w_codes, x_codes (N, K), (M, K) int8, 16-byte aligned; w_scales, x_scales their fp16 scales
+ *   the rest     as for ksd_w8a8_gemm_nt_ex
+ */
+int ksd_int8_linear(const void *x, int x_dtype, int64_t M, int64_t x_stride, const float *w,
+                    int64_t N, int64_t K, int8_t *w_codes, uint16_t *w_scales, int8_t *x_codes,
+                    uint16_t *x_scales, const float *bias, const void *residual, void *y,
+                    int y_dtype, float *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * Q2 — dequantize along the last dim: out = float(code) * float(scale) per group.
  * Replaces dequantize_last_dim (reference ksdraft/kernels/quant.py:55-67).
  *   codes (rows, K) int8; scales (rows, n_scales) fp16; out (rows, K) fp32.

@@ -87,13 +87,13 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(
 // past num_records, so no store sits in a branch and no wait covers the stores.
 // Requires K % 8 == 0, 16-byte aligned rows and 8-byte aligned code rows.
 template <int DT, int G, int RT>
-__global__ __launch_bounds__(256) void quant_rows_fast_kernel(
+__device__ __forceinline__ void quant_rows_fast(
     const void *__restrict__ xv, int64_t rows, int K, int64_t stride, int ngroups,
-    int8_t *__restrict__ codes, uint16_t *__restrict__ scales) {
+    int8_t *__restrict__ codes, uint16_t *__restrict__ scales, unsigned bx) {
   using T = typename Elem<DT>::T;
   constexpr int LPG = G / 8;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t row0 = ((int64_t)blockIdx.x * 4 + wave) * RT;
+  const int64_t row0 = ((int64_t)bx * 4 + wave) * RT;
   if (row0 >= rows) return;                                   // wave-uniform
   const int k0 = ((int)blockIdx.y * 64 + (int)(threadIdx.x & 63)) * 8;
   const bool kok = k0 < K;
@@ -119,6 +119,28 @@ __global__ __launch_bounds__(256) void quant_rows_fast_kernel(
     __builtin_amdgcn_raw_buffer_store_b16(scale_bits(s), rsrc(scales + row * ngroups, 2 * (int64_t)ngroups),
                                           lead ? (uint32_t)(k0 / G) * 2 : kOob, 0, 0);
   }
+}
+
+template <int DT, int G, int RT>
+__global__ __launch_bounds__(256) void quant_rows_fast_kernel(
+    const void *__restrict__ xv, int64_t rows, int K, int64_t stride, int ngroups,
+    int8_t *__restrict__ codes, uint16_t *__restrict__ scales) {
+  quant_rows_fast<DT, G, RT>(xv, rows, K, stride, ngroups, codes, scales, blockIdx.x);
+}
+
+// Both operands of an int8 linear in one launch: the first nbw blocks of a row slice take the fp32
+// master W, the others x. A decode call is bound by its launches (the two quantizations of 16 x 1536
+// tokens and 1536 x 1536 weights take 2.7 and 4.3 us of device time, a launch about as long on the host):
+// that call went from 60.4 to 32.1 us with this launch, the few-row GEMM and one entry for the three.
+template <int DT, int RTW, int RTX>
+__global__ __launch_bounds__(256) void quant_rows_pair_kernel(
+    const float *__restrict__ w, int64_t N, int8_t *__restrict__ wcodes, uint16_t *__restrict__ wscales,
+    unsigned nbw, const void *__restrict__ x, int64_t M, int64_t xstride, int8_t *__restrict__ xcodes,
+    uint16_t *__restrict__ xscales, int K, int ngroups) {
+  if (blockIdx.x < nbw)
+    quant_rows_fast<KSD_F32, 128, RTW>(w, N, K, K, ngroups, wcodes, wscales, blockIdx.x);
+  else
+    quant_rows_fast<DT, 128, RTX>(x, M, K, xstride, ngroups, xcodes, xscales, blockIdx.x - nbw);
 }
 
 // ----------------------------------------------------------------------------------
@@ -849,15 +871,17 @@ static int launch_quant_T(const void *x, const uint16_t *in_scales, int64_t nsc_
   return check_launch("quantize_transpose");
 }
 
+// Four rows per wave where that still gives every CU several blocks.
+static bool four_rows(int64_t rows, int64_t K) { return cdiv(rows, 16) * cdiv(K, 512) >= 1024; }
+
 template <int DT, int G>
 static void launch_rows(const void *x, int64_t rows, int64_t K, int64_t stride,
                         int8_t *codes, uint16_t *scales, const float *noise, float d2,
                         bool vec, hipStream_t st) {
   const int64_t ng = cdiv(K, G);
   if (vec && noise == nullptr && K <= (1 << 24)) {
-    // four rows per wave where that still gives every CU several blocks
     const unsigned gy = (unsigned)cdiv(K, 512);
-    if (cdiv(rows, 16) * gy >= 1024) {
+    if (four_rows(rows, K)) {
       const dim3 grid((unsigned)cdiv(rows, 16), gy);
       quant_rows_fast_kernel<DT, G, 4><<<grid, 256, 0, st>>>(x, rows, (int)K, stride, (int)ng, codes, scales);
     } else {
@@ -1022,6 +1046,47 @@ extern "C" int ksd_quantize_lastdim(const void *x, int x_dtype, int64_t rows, in
     default: return fail(KSD_ETYPE, "quantize expects float32, bfloat16 or float16 input");
   }
   return check_launch("quantize_lastdim");
+}
+
+extern "C" int ksd_int8_linear(const void *x, int x_dtype, int64_t M, int64_t x_stride, const float *w, int64_t N,
+                               int64_t K, int8_t *w_codes, uint16_t *w_scales, int8_t *x_codes, uint16_t *x_scales,
+                               const float *bias, const void *residual, void *y, int y_dtype, float *workspace,
+                               int64_t workspace_bytes, void *stream) {
+  if (K % 128 != 0 || K <= 0) return fail(KSD_EINVAL, "int8_linear: K=%lld must be a positive multiple of 128", (long long)K);
+  if (M < 0 || N < 0 || x_stride < K) return fail(KSD_EINVAL, "bad int8_linear shape");
+  const int esz = x_dtype == KSD_F32 ? 4 : 2;
+  const bool vec = ((uintptr_t)x | (uintptr_t)w) % 16 == 0 && (x_stride * esz) % 16 == 0 && K <= (1 << 24) &&
+                   ((uintptr_t)w_codes | (uintptr_t)x_codes) % 8 == 0;
+  const int rtw = four_rows(N, K) ? 4 : 1, rtx = four_rows(M, K) ? 4 : 1;
+  const int64_t nbw = cdiv(N, 4 * rtw), nbx = cdiv(M, 4 * rtx);
+  if (vec && M > 0 && N > 0 && nbw + nbx <= 0x7fffffffLL) {
+    const dim3 grid((unsigned)(nbw + nbx), (unsigned)cdiv(K, 512));
+    hipStream_t st = (hipStream_t)stream;
+#define KSD_PAIR(DT, RW, RX)                                                                                       \
+  quant_rows_pair_kernel<DT, RW, RX><<<grid, 256, 0, st>>>(w, N, w_codes, w_scales, (unsigned)nbw, x, M, x_stride, \
+                                                           x_codes, x_scales, (int)K, (int)(K / 128))
+#define KSD_PAIR_DT(DT)                                                                  \
+  if (rtw == 4 && rtx == 4) KSD_PAIR(DT, 4, 4);                                          \
+  else if (rtw == 4) KSD_PAIR(DT, 4, 1);                                                 \
+  else if (rtx == 4) KSD_PAIR(DT, 1, 4);                                                 \
+  else KSD_PAIR(DT, 1, 1);
+    switch (x_dtype) {
+      case KSD_F32: KSD_PAIR_DT(KSD_F32); break;
+      case KSD_BF16: KSD_PAIR_DT(KSD_BF16); break;
+      case KSD_F16: KSD_PAIR_DT(KSD_F16); break;
+      default: return fail(KSD_ETYPE, "quantize expects float32, bfloat16 or float16 input");
+    }
+#undef KSD_PAIR_DT
+#undef KSD_PAIR
+    const int rc = check_launch("int8_linear");
+    if (rc) return rc;
+  } else {  // unaligned rows: a launch each
+    int rc = ksd_quantize_lastdim(w, KSD_F32, N, K, K, 128, w_codes, w_scales, nullptr, 0.0f, stream);
+    if (!rc) rc = ksd_quantize_lastdim(x, x_dtype, M, K, x_stride, 128, x_codes, x_scales, nullptr, 0.0f, stream);
+    if (rc) return rc;
+  }
+  return ksd_w8a8_gemm_nt_ex(x_codes, x_scales, w_codes, w_scales, M, N, K, 128, bias, residual, y, y_dtype,
+                             workspace, workspace_bytes, stream);
 }
 
 // ----------------------------------------------------------------------------------

@@ -21,8 +21,9 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from .gemm import w8a8_gemm, w8a8_gemm_out, w8a8_gemm_pair
-from .quant import (GROUP_SIZE, dequantize_last_dim, quantize_dual, quantize_dual2,
+from .. import _lib
+from .gemm import gemm_splits, w8a8_gemm, w8a8_gemm_out, w8a8_gemm_pair
+from .quant import (GROUP_SIZE, SCALE_DTYPE, dequantize_last_dim, quantize_dual, quantize_dual2,
                     quantize_dual_colsum, quantize_last_dim, quantize_last_dim_dithered,
                     quantize_transpose, requant_transpose)
 
@@ -46,6 +47,41 @@ def w8a8_linear_forward(x2: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor,
     y = w8a8_gemm_out(xq, xs, wq, ws, group, bias=bias,
                       out_dtype=_out_dtype(out_dtype or x2.dtype), residual=residual)
     return y, xq, xs
+
+
+def w8a8_linear_master(x2: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None,
+                       residual: torch.Tensor | None = None):
+    """w8a8_linear_forward from the fp32 master, its quantization in the launch that
+    quantizes x2 (ksd_int8_linear): (y, weight codes, weight scales), or None where that
+    entry does not apply (K no multiple of 128, empty or other operands)."""
+    M, K = x2.shape
+    if (w.dtype != torch.float32 or w.dim() != 2 or w.shape[1] != K or K == 0 or K % GROUP_SIZE
+            or M == 0 or not w.is_contiguous() or x2.dtype not in _OUT_DTYPES or not x2.is_cuda):
+        return None
+    N = w.shape[0]
+    if (N == 0 or (bias is not None and (bias.dtype != torch.float32 or not bias.is_contiguous()
+                                         or bias.numel() != N or bias.device != x2.device))
+            or (residual is not None and (residual.shape != (M, N) or residual.dtype != x2.dtype
+                                          or residual.device != x2.device))):
+        return None
+    dev = _lib.require_gpu(x2, w)
+    if x2.stride(1) != 1 or (M > 1 and x2.stride(0) < K):
+        x2 = x2.contiguous()
+    if residual is not None:
+        residual = residual.contiguous()
+    G = K // GROUP_SIZE
+    wq = torch.empty((N, K), dtype=torch.int8, device=dev)
+    ws = torch.empty((N, G), dtype=SCALE_DTYPE, device=dev)
+    xq = torch.empty(M * (K + 2 * G), dtype=torch.int8, device=dev)  # x's codes, then its scales
+    y = torch.empty((M, N), dtype=x2.dtype, device=dev)
+    splits = gemm_splits(M, N, K)
+    work = torch.empty(splits * M * N, dtype=torch.float32, device=dev) if splits > 1 else None
+    _lib.call("ksd_int8_linear", x2.data_ptr(), _lib.dtype_code(x2.dtype), M,
+              x2.stride(0) if M > 1 else K, w.data_ptr(), N, K, wq.data_ptr(), ws.data_ptr(),
+              xq.data_ptr(), xq.data_ptr() + M * K, _lib.ptr(bias), _lib.ptr(residual),
+              y.data_ptr(), _lib.dtype_code(y.dtype), _lib.ptr(work),
+              0 if work is None else work.numel() * 4, _lib.stream_ptr(dev))
+    return y, wq, ws
 
 
 def w8a8_linear_forward_train(x2: torch.Tensor, wq: torch.Tensor, ws: torch.Tensor,
@@ -252,9 +288,23 @@ class Int8Linear(nn.Module):
         train = torch.is_grad_enabled() and (self.weight.requires_grad or x.requires_grad
                                              or (residual is not None and residual.requires_grad))
         xpre = None
+        fuse_res = (residual is not None and x.dtype in _OUT_DTYPES
+                    and residual.dtype == x.dtype and not self.ste_training)
         if not self._codes_current():
             self._codes_key = None
             w = self.weight.detach()
+            if (not train and float(getattr(self, "_dither", 0.0)) <= 0.0
+                    and not (self.training and self.weight.requires_grad)):
+                # eval: the master's codes, x's codes and the GEMM in one call
+                out = w8a8_linear_master(
+                    x.reshape(-1, x.shape[-1]), w,
+                    None if self.bias is None else self.bias.detach(),
+                    residual.reshape(-1, self.out_features) if fuse_res else None)
+                if out is not None:
+                    y, self.weight_codes, self.weight_scales = out
+                    self._wt, self._wt_src = None, self.weight_codes
+                    y = y.reshape(*x.shape[:-1], self.out_features)
+                    return y if fuse_res or residual is None else residual + y
             if (train and not self.ste_training and self.training and self.weight.requires_grad
                     and float(getattr(self, "_dither", 0.0)) == 0.0 and w.dim() == 2
                     and w.dtype == torch.float32 and x.dtype == torch.float32):
@@ -265,8 +315,6 @@ class Int8Linear(nn.Module):
                 self._wt, self._wt_src = (ct, st), codes
             else:
                 self._quantize_weight()
-        fuse_res = (residual is not None and x.dtype in _OUT_DTYPES
-                    and residual.dtype == x.dtype and not self.ste_training)
         if train:
             if self.ste_training:
                 y = self.fake_quant_forward(x)
