@@ -122,30 +122,62 @@ def check(status: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args))
+    status = getattr(_lib or load(), name)(*args)
+    if status:
+        check(status)
 
 
 def require_gpu(*tensors: torch.Tensor) -> torch.device:
     """All tensors must live on one HIP device; returns it."""
-    dev = None
+    dev = index = None
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "ksdraft_amd kernels run on the GPU only (no CPU path); got a tensor on "
                 f"{t.device}")
         if dev is None:
-            dev = t.device
-        elif t.device != dev:
+            dev, index = t.device, t.get_device()
+        elif t.get_device() != index:
             raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
     if dev is None:
         raise RuntimeError("no tensor given")
     return dev
 
 
+# The current stream's handle without the torch.cuda.Stream object around it, which costs 4 us a
+# call, as much as the launch (a torch built without the raw getter goes through the object).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    if _raw_stream is None or dev.index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(dev.index)
+
+
+def put(module: torch.nn.Module, **values) -> None:
+    """module.name = value for registered buffers and for plain attributes, without the walk
+    through nn.Module.__setattr__ (3 to 4 us each, a dozen of them per training call). Names
+    that are neither yet, values under a buffer registration hook and classes with a
+    __setattr__ of their own take that walk."""
+    if type(module).__setattr__ is not torch.nn.Module.__setattr__:
+        for name, value in values.items():
+            setattr(module, name, value)
+        return
+    attrs = module.__dict__
+    buffers = attrs["_buffers"]
+    for name, value in values.items():
+        if name in attrs:
+            attrs[name] = value
+        elif name in buffers and not _buffer_hooks:
+            buffers[name] = value
+        else:
+            setattr(module, name, value)
+
+
+_buffer_hooks = getattr(torch.nn.modules.module, "_global_buffer_registration_hooks", {})
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

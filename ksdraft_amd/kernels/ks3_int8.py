@@ -421,20 +421,21 @@ class KS3Int8Cell(nn.Module):
     def _repack_masters(self):
         """ks3_int8.py:262-277. The down/up codes are skipped when the optimizer already
         wrote them from the masters as they are (the same quantize_last_dim)."""
+        put = _lib.put
         if not self._master_codes_current("down"):
-            self.down_codes, self.down_scales = quantize_last_dim(self.master_down, self.group)
+            codes, scales = quantize_last_dim(self.master_down, self.group)
+            put(self, down_codes=codes, down_scales=scales)
         if not self._master_codes_current("up"):
-            self.up_codes, self.up_scales = quantize_last_dim(self.master_up, self.group)
+            codes, scales = quantize_last_dim(self.master_up, self.group)
+            put(self, up_codes=codes, up_scales=scales)
         sq, ss = pack_spine(self.master_coefficients, self.group)
-        self.spine_codes, self.spine_scale = sq, ss
         scale_t = F.softplus(self.master_raw_scale.detach()) + 1e-4
         shift_t = 0.5 * torch.tanh(self.master_raw_shift.detach())
         wsc, wss = quantize_last_dim(scale_t.reshape(-1, 1), self.group)
         whc, whs = quantize_last_dim(shift_t.reshape(-1, 1), self.group)
-        self.warp_scale_codes, self.warp_scale_scales = wsc, wss
-        self.warp_shift_codes, self.warp_shift_scales = whc, whs
-        self.warp_scale_raw = self.master_raw_scale.detach()
-        self.warp_shift_raw = self.master_raw_shift.detach()
+        put(self, spine_codes=sq, spine_scale=ss, warp_scale_codes=wsc, warp_scale_scales=wss,
+            warp_shift_codes=whc, warp_shift_scales=whs,
+            warp_scale_raw=self.master_raw_scale.detach(), warp_shift_raw=self.master_raw_shift.detach())
 
     def _out_dtype(self, x):
         return (torch.get_autocast_gpu_dtype()

@@ -238,10 +238,8 @@ class Int8Linear(nn.Module):
             wt = (ct, st)
         else:
             codes, scales = quantize_last_dim(w.float())
-        self.weight_codes = codes
-        self.weight_scales = scales
-        self._wt = wt  # valid while weight_codes is these codes
-        self._wt_src = codes
+        # _wt is valid while weight_codes is these codes
+        _lib.put(self, weight_codes=codes, weight_scales=scales, _wt=wt, _wt_src=codes)
 
     def _quantize_weight_dithered(self, dither: float) -> None:
         self._dither = dither
@@ -251,7 +249,7 @@ class Int8Linear(nn.Module):
         """Forget codes handed over by an optimizer (train.AdamWRequant.register_int8):
         the next call requantizes the master. Needed after a write to the master that
         torch does not version, i.e. through ``weight.data`` or a raw pointer."""
-        self._codes_key = None
+        _lib.put(self, _codes_key=None)
 
     def _codes_current(self) -> bool:
         """True when train.AdamWRequant wrote the codes in the same pass that last
@@ -291,7 +289,7 @@ class Int8Linear(nn.Module):
         fuse_res = (residual is not None and x.dtype in _OUT_DTYPES
                     and residual.dtype == x.dtype and not self.ste_training)
         if not self._codes_current():
-            self._codes_key = None
+            _lib.put(self, _codes_key=None)
             w = self.weight.detach()
             if (not train and float(getattr(self, "_dither", 0.0)) <= 0.0
                     and not (self.training and self.weight.requires_grad)):
@@ -301,8 +299,8 @@ class Int8Linear(nn.Module):
                     None if self.bias is None else self.bias.detach(),
                     residual.reshape(-1, self.out_features) if fuse_res else None)
                 if out is not None:
-                    y, self.weight_codes, self.weight_scales = out
-                    self._wt, self._wt_src = None, self.weight_codes
+                    y, codes, scales = out
+                    _lib.put(self, weight_codes=codes, weight_scales=scales, _wt=None, _wt_src=codes)
                     y = y.reshape(*x.shape[:-1], self.out_features)
                     return y if fuse_res or residual is None else residual + y
             if (train and not self.ste_training and self.training and self.weight.requires_grad
@@ -311,8 +309,7 @@ class Int8Linear(nn.Module):
                 # a training forward quantizes the master (both layouts) and x (both
                 # layouts) in one launch
                 (codes, scales, ct, st), xpre = quantize_dual2(w, x.reshape(-1, x.shape[-1]))
-                self.weight_codes, self.weight_scales = codes, scales
-                self._wt, self._wt_src = (ct, st), codes
+                _lib.put(self, weight_codes=codes, weight_scales=scales, _wt=(ct, st), _wt_src=codes)
             else:
                 self._quantize_weight()
         if train:

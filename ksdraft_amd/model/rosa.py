@@ -17,6 +17,7 @@ import torch
 from torch import nn
 from torch.nn import functional as F
 
+from .. import _lib
 from ..kernels import rosa as R
 
 
@@ -93,7 +94,7 @@ class RosaMixer(nn.Module):
         for p in projs:
             assert isinstance(p, Int8Linear)
             if not p._codes_current():  # as Int8Linear.forward: live masters stay authoritative
-                p._codes_key = None
+                _lib.put(p, _codes_key=None)
                 p._quantize_weight()
             args += [p.weight, p.bias, p.weight_codes, p.weight_scales]
         sig = [torch.sigmoid(m) for m in mixes]

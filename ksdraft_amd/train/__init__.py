@@ -330,11 +330,9 @@ class AdamWRequant(torch.optim.Optimizer):
                 mod, name = reg
                 key = (p.data_ptr(), p._version)
                 if name is None:
-                    mod.weight_codes, mod.weight_scales = res
-                    mod._codes_key = key
+                    _lib.put(mod, weight_codes=res[0], weight_scales=res[1], _codes_key=key)
                 else:
-                    setattr(mod, name + "_codes", res[0])
-                    setattr(mod, name + "_scales", res[1])
+                    _lib.put(mod, **{name + "_codes": res[0], name + "_scales": res[1]})
                     mod._master_codes_keys[name] = key
                 if self.build_transposes and mod.training and res[0].dim() == 2:
                     tpairs.append(res)
@@ -342,7 +340,7 @@ class AdamWRequant(torch.optim.Optimizer):
             # the dX operands W^T of the next backward, for all masters in a few launches
             for (mod, name, codes), wt in zip(towners, requant_transpose_multi(tpairs)):
                 if name is None:
-                    mod._wt, mod._wt_src = wt, codes
+                    _lib.put(mod, _wt=wt, _wt_src=codes)
                 else:
                     if getattr(mod, "_master_t", None) is None:
                         mod._master_t = {}

@@ -112,3 +112,34 @@ def test_int8_linear_codes_follow_writes_the_optimizer_did_not_make():
     lin2.weight_codes, lin2.weight_scales = lin.weight_codes, lin.weight_scales
     lin2._codes_key = (lin2.weight.data_ptr(), lin2.weight._version)
     assert not lin2._codes_current()
+
+
+def test_put_assigns_as_setattr_does():
+    """_lib.put: buffers, plain attributes, new names, a registration hook and a class with its
+    own __setattr__ end as module.name = value leaves them."""
+    from ksdraft_amd import _lib
+
+    class Own(torch.nn.Linear):
+        def __setattr__(self, name, value):
+            super().__setattr__(name, value)
+            if name == "codes":
+                self.__dict__["seen"] = value
+
+    t = torch.zeros(2)
+    for cls in (torch.nn.Linear, Own):
+        a, b = cls(2, 2), cls(2, 2)
+        for m in (a, b):
+            m.register_buffer("codes", None, persistent=False)
+            m.plain = None
+        _lib.put(a, codes=t, plain=(t,), fresh=1)
+        b.codes, b.plain, b.fresh = t, (t,), 1
+        assert list(a.state_dict()) == list(b.state_dict()) and dict(a.named_buffers()).keys() == dict(b.named_buffers()).keys()
+        assert a.codes is t and a.plain == (t,) and a.fresh == 1
+        assert getattr(a, "seen", None) is getattr(b, "seen", None)
+    calls = []
+    h = torch.nn.modules.module.register_module_buffer_registration_hook(lambda m, n, v: calls.append(n))
+    try:
+        _lib.put(a, codes=t)
+    finally:
+        h.remove()
+    assert calls == ["codes"]
