@@ -511,6 +511,25 @@ int ksd_rosa_shift_quant(const void *x, int x_dtype, int64_t B, int64_t T, int64
                          int8_t *v_codes, uint16_t *v_scales, void *stream);
 
 /*
+ * R1 and the three int8 projections of an eval mixer (reference ksdraft/model/rosa.py:128-149
+ * with Int8Linear, ksdraft/kernels/linear.py:62-73): sigmoid(mix) and the codes of the three
+ * fp32 masters in one launch, ksd_rosa_shift_quant, then the three GEMMs (+ bias), in one launch
+ * where each would take the few-row kernel. The same outputs as those calls one by one.
+ *   x        (B, T, d) of type x_dtype, dense; d a positive multiple of 128
+ *   mix, w, bias, w_codes, w_scales, y: three pointers each (q, k, v): (d,) fp32, (S, d) fp32,
+ *            (S,) fp32 or NULL (bias itself may be NULL), (S, d) int8 16-byte aligned,
+ *            (S, d/128) fp16, (B*T, S) of type x_dtype
+ *   sig      (3, d) fp32, 16-byte aligned; x_codes (3, B*T, d) int8, 16-byte aligned;
+ *   x_scales (3, B*T, d/128) fp16: all three written
+ *   workspace as for ksd_w8a8_gemm_nt_ex (one GEMM's, B*T x S x d)
+ */
+int ksd_rosa_projections(const void *x, int x_dtype, int64_t B, int64_t T, int64_t d,
+                         const float *const *mix, const float *const *w, int64_t S,
+                         const float *const *bias, int8_t *const *w_codes, uint16_t *const *w_scales,
+                         float *sig, int8_t *x_codes, uint16_t *x_scales, void *const *y,
+                         float *workspace, int64_t workspace_bytes, void *stream);
+
+/*
  * R1, training form — RosaMixer._shifted (reference ksdraft/model/rosa.py:128-133) fused
  * with the training quantization of each projection input: the row codes of the forward
  * GEMM (Int8Linear, ksdraft/kernels/linear.py:69) and dW's operand, the input transposed and

@@ -68,6 +68,9 @@ int ks3_fused_table(const int8_t *spine_codes, const uint16_t *spine_scale, cons
 bool rows_gemm_fits(int64_t M, int64_t N, int64_t K);
 void rows_gemm(const int8_t *a, const uint16_t *as, const int8_t *w, const uint16_t *ws, int M, int N, int K,
                int splits, const float *bias, const void *residual, void *y, int out, hipStream_t st);
+void rows_gemm3(const int8_t *const a[3], const uint16_t *const as[3], const int8_t *const w[3],
+                const uint16_t *const ws[3], int M, int N, int K, int splits, const float *const bias[3],
+                void *const y[3], int out, hipStream_t st);
 
 // ---------------------------------------------------------------- device numerics
 constexpr float kScaleMin = 5.9604644775390625e-08f;  // 2**-24, quant.py:22

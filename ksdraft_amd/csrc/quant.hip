@@ -143,6 +143,39 @@ __global__ __launch_bounds__(256) void quant_rows_pair_kernel(
     quant_rows_fast<DT, 128, RTX>(x, M, K, xstride, ngroups, xcodes, xscales, blockIdx.x - nbw);
 }
 
+// What a mixer's eval projections need besides x, in one launch: the row codes of the three fp32
+// masters (blocks below end[2]) and sigmoid(mix) of the three mixes (the rest; the formula and the
+// library functions of torch.sigmoid, so the same bits). Six launches of 2 to 4 us on a path that is
+// bound by its launches. 1 x 301 x 1536 -> 3 x 512: 4.7 us of
+// device time where the six took 16.2; with the batched GEMM and one output pass the mixer's call went
+// from 221 to 127 us.
+struct MixPrep {
+  const float *w[3];
+  int8_t *codes[3];
+  uint16_t *scales[3];
+  int64_t N[3];
+  unsigned end[3];  // first block past each master
+  const float *mix[3];
+  float *sig;       // (3, K)
+};
+template <int RT>
+__global__ __launch_bounds__(256) void mix_prep_kernel(const MixPrep a, int K, int ngroups) {
+  unsigned first = 0;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    if (blockIdx.x < a.end[j]) {
+      quant_rows_fast<KSD_F32, 128, RT>(a.w[j], a.N[j], K, K, ngroups, a.codes[j], a.scales[j], blockIdx.x - first);
+      return;
+    }
+    first = a.end[j];
+  }
+  const int i = (int)(blockIdx.x - first) * 256 + (int)threadIdx.x;
+  if (blockIdx.y != 0 || i >= 3 * K) return;
+  const int j = i / K;
+  const float *m = j == 0 ? a.mix[0] : j == 1 ? a.mix[1] : a.mix[2];
+  a.sig[i] = 1.0f / (1.0f + expf(-m[i - j * K]));
+}
+
 // ----------------------------------------------------------------------------------
 // Dequantization: out = float(code) * float(scale), exact in fp32 (quant.py:66).
 __global__ __launch_bounds__(256) void dequant_rows_kernel(
@@ -1054,6 +1087,8 @@ extern "C" int ksd_int8_linear(const void *x, int x_dtype, int64_t M, int64_t x_
                                int64_t workspace_bytes, void *stream) {
   if (K % 128 != 0 || K <= 0) return fail(KSD_EINVAL, "int8_linear: K=%lld must be a positive multiple of 128", (long long)K);
   if (M < 0 || N < 0 || x_stride < K) return fail(KSD_EINVAL, "bad int8_linear shape");
+  if (M > 0 && N > 0 && (!x || !w || !w_codes || !w_scales || !x_codes || !x_scales || !y))
+    return fail(KSD_EINVAL, "int8_linear: null pointer");
   const int esz = x_dtype == KSD_F32 ? 4 : 2;
   const bool vec = ((uintptr_t)x | (uintptr_t)w) % 16 == 0 && (x_stride * esz) % 16 == 0 && K <= (1 << 24) &&
                    ((uintptr_t)w_codes | (uintptr_t)x_codes) % 8 == 0;
@@ -1087,6 +1122,76 @@ extern "C" int ksd_int8_linear(const void *x, int x_dtype, int64_t M, int64_t x_
   }
   return ksd_w8a8_gemm_nt_ex(x_codes, x_scales, w_codes, w_scales, M, N, K, 128, bias, residual, y, y_dtype,
                              workspace, workspace_bytes, stream);
+}
+
+extern "C" int ksd_rosa_projections(const void *x, int x_dtype, int64_t B, int64_t T, int64_t d,
+                                    const float *const *mix, const float *const *w, int64_t S,
+                                    const float *const *bias, int8_t *const *w_codes, uint16_t *const *w_scales,
+                                    float *sig, int8_t *x_codes, uint16_t *x_scales, void *const *y,
+                                    float *workspace, int64_t workspace_bytes, void *stream) {
+  if (B < 0 || T < 0 || S < 0) return fail(KSD_EINVAL, "rosa_projections: negative shape");
+  if (d <= 0 || d % 128 != 0 || d > (1 << 24))
+    return fail(KSD_EINVAL, "rosa_projections: d=%lld must be a positive multiple of 128", (long long)d);
+  if (x_dtype != KSD_F32 && x_dtype != KSD_BF16 && x_dtype != KSD_F16)
+    return fail(KSD_ETYPE, "rosa_projections: x must be float32, bfloat16 or float16");
+  if (B == 0 || T == 0 || S == 0) return KSD_OK;
+  if (T > 0x7fffffffLL || B > (0x7fffffffLL - 64) / T || S > 0x7fffffffLL / 3)
+    return fail(KSD_EINVAL, "rosa_projections: too large");
+  if (!x || !mix || !w || !w_codes || !w_scales || !sig || !x_codes || !x_scales || !y)
+    return fail(KSD_EINVAL, "rosa_projections: null pointer");
+  const int64_t M = B * T, G = d / 128;
+  bool vec = true;
+  for (int i = 0; i < 3; ++i) {
+    if (!mix[i] || !w[i] || !w_codes[i] || !w_scales[i] || !y[i])
+      return fail(KSD_EINVAL, "rosa_projections: null pointer");
+    if ((((uintptr_t)w_codes[i] | (uintptr_t)x_codes) & 15) != 0)
+      return fail(KSD_EINVAL, "rosa_projections: codes must be 16-byte aligned");
+    vec = vec && ((uintptr_t)w[i] & 15) == 0;
+  }
+  int splits = 1;
+  int rc = ksd_w8a8_gemm_splits(M, S, d, 128, &splits);
+  if (rc) return rc;
+  const bool rows = rows_gemm_fits(M, S, d);
+  const int64_t need = splits > 1 && !rows ? (int64_t)splits * M * S * 4 : 0;
+  if (need > 0 && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0))
+    return fail(KSD_EINVAL, "rosa_projections: needs a 16-byte aligned fp32 workspace of %lld bytes", (long long)need);
+  hipStream_t st = (hipStream_t)stream;
+  MixPrep p{};
+  const int rt = four_rows(3 * S, d) ? 4 : 1;
+  for (int i = 0; i < 3; ++i) {
+    if (!vec) {  // unaligned masters: a launch each
+      rc = ksd_quantize_lastdim(w[i], KSD_F32, S, d, d, 128, w_codes[i], w_scales[i], nullptr, 0.0f, stream);
+      if (rc) return rc;
+    }
+    p.w[i] = w[i];
+    p.codes[i] = w_codes[i];
+    p.scales[i] = w_scales[i];
+    p.N[i] = S;
+    p.end[i] = vec ? (unsigned)((i + 1) * cdiv(S, 4 * rt)) : 0;
+    p.mix[i] = mix[i];
+  }
+  p.sig = sig;
+  const dim3 grid(p.end[2] + (unsigned)cdiv(3 * d, 256), vec ? (unsigned)cdiv(d, 512) : 1u);
+  if (rt == 4) mix_prep_kernel<4><<<grid, 256, 0, st>>>(p, (int)d, (int)G);
+  else mix_prep_kernel<1><<<grid, 256, 0, st>>>(p, (int)d, (int)G);
+  if ((rc = check_launch("rosa_projections"))) return rc;
+  int8_t *xc[3] = {x_codes, x_codes + M * d, x_codes + 2 * M * d};
+  uint16_t *xs[3] = {x_scales, x_scales + M * G, x_scales + 2 * M * G};
+  rc = ksd_rosa_shift_quant(x, x_dtype, B, T, d, sig, sig + d, sig + 2 * d, 128, xc[0], xs[0], xc[1], xs[1], xc[2],
+                            xs[2], stream);
+  if (rc) return rc;
+  const float *none[3] = {nullptr, nullptr, nullptr};
+  if (!bias) bias = none;
+  if (rows) {  // each would take the few-row kernel: all three in one launch of it
+    rows_gemm3(xc, xs, w_codes, w_scales, (int)M, (int)S, (int)d, splits, bias, y, x_dtype, st);
+    return check_launch("rosa_projections");
+  }
+  for (int i = 0; i < 3; ++i) {
+    rc = ksd_w8a8_gemm_nt_ex(xc[i], xs[i], w_codes[i], w_scales[i], M, S, d, 128, bias[i], nullptr, y[i], x_dtype,
+                             workspace, workspace_bytes, stream);
+    if (rc) return rc;
+  }
+  return KSD_OK;
 }
 
 // ----------------------------------------------------------------------------------

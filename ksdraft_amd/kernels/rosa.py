@@ -2,6 +2,7 @@
 ksdraft/model/rosa.py and ksdraft/kernels/rosa_credit_gpu.py).
 
   shift_quantize   RosaMixer._shifted fused with each projection input's quantization
+  shift_project    the same and the three eval projections behind it, in one call
   shift_quantize_dual   the same for training: row codes plus dW's transposed operand
   shift_backward   the shift's backward: the input gradient and the sigmoid(mix) gradients
   ShiftedInt8Projections   autograd of shift + the three Int8Linear q/k/v projections
@@ -17,6 +18,7 @@ import ctypes
 import torch
 
 from .. import _lib
+from .gemm import gemm_splits
 from .quant import GROUP_SIZE, SCALE_DTYPE
 
 
@@ -50,6 +52,42 @@ def shift_quantize(x: torch.Tensor, sig_q: torch.Tensor, sig_k: torch.Tensor,
               outs[1][1].data_ptr(), outs[2][0].data_ptr(), outs[2][1].data_ptr(),
               _lib.stream_ptr(dev))
     return tuple(outs)
+
+
+def shift_project(x: torch.Tensor, mixes, weights, biases):
+    """The q, k and v projections of an eval mixer on live fp32 masters (ksd_rosa_projections):
+    ([(B, T, S)] * 3, [(weight codes, scales)] * 3), or None where that entry does not apply
+    (d no multiple of 128, empty, other types, shapes or layouts)."""
+    d = x.shape[-1]
+    S = weights[0].shape[0]
+    f32 = torch.float32
+    ok = (x.is_cuda and x.dim() == 3 and x.numel() > 0 and d % GROUP_SIZE == 0 and S > 0
+          and x.dtype in (f32, torch.bfloat16, torch.float16)
+          and all(m.dtype == f32 and m.shape == (d,) and m.is_contiguous() for m in mixes)
+          and all(w.dtype == f32 and w.shape == (S, d) and w.is_contiguous() for w in weights)
+          and all(b is None or (b.dtype == f32 and b.shape == (S,) and b.is_contiguous()) for b in biases)
+          and x.shape[0] * x.shape[1] < 2 ** 31 - 64 and d <= 1 << 24 and S < 2 ** 31 // 3)
+    if not ok:
+        return None
+    dev = _lib.require_gpu(x, *mixes, *weights, *biases)
+    x = x.contiguous()
+    B, T, _ = x.shape
+    M, G = B * T, d // GROUP_SIZE
+    codes = [(torch.empty((S, d), dtype=torch.int8, device=dev),
+              torch.empty((S, G), dtype=SCALE_DTYPE, device=dev)) for _ in range(3)]
+    ys = [torch.empty((B, T, S), dtype=x.dtype, device=dev) for _ in range(3)]
+    # sigmoid(mix), then the inputs' codes and their scales
+    tmp = torch.empty(3 * (4 * d + M * (d + 2 * G)), dtype=torch.int8, device=dev)
+    at = tmp.data_ptr()
+    splits = gemm_splits(M, S, d)
+    work = torch.empty(splits * M * S, dtype=f32, device=dev) if splits > 1 else None
+    _lib.call("ksd_rosa_projections", x.data_ptr(), _lib.dtype_code(x.dtype), B, T, d,
+              _ptr_array([m.data_ptr() for m in mixes]), _ptr_array([w.data_ptr() for w in weights]), S,
+              _ptr_array([_lib.ptr(b) for b in biases]), _ptr_array([c.data_ptr() for c, _ in codes]),
+              _ptr_array([s.data_ptr() for _, s in codes]), at, at + 12 * d, at + 12 * d + 3 * M * d,
+              _ptr_array([y.data_ptr() for y in ys]), _lib.ptr(work),
+              0 if work is None else work.numel() * 4, _lib.stream_ptr(dev))
+    return ys, codes
 
 
 def _ptr_array(ptrs):

@@ -105,12 +105,23 @@ class RosaMixer(nn.Module):
         """Eval with Int8Linear q/k/v: shift + quantize in one pass, then the W8A8 GEMMs
         (+ bias) exactly as Int8Linear.forward computes them (linear.py:62-73)."""
         from ..kernels.gemm import w8a8_gemm_out
+        projs = (self.q_proj, self.k_proj, self.v_proj)
+        if not any(float(getattr(p, "_dither", 0.0)) > 0.0 or (p.training and p.weight.requires_grad)
+                   for p in projs):
+            out = R.shift_project(
+                x, [m.detach() for m in (self.time_mix_q, self.time_mix_k, self.time_mix_v)],
+                [p.weight.detach() for p in projs],
+                [None if p.bias is None else p.bias.detach() for p in projs])
+            if out is not None:
+                for p, (codes, scales) in zip(projs, out[1]):
+                    _lib.put(p, weight_codes=codes, weight_scales=scales, _wt=None, _wt_src=codes)
+                return out[0]
         sig = [torch.sigmoid(m.detach().float()) for m in (self.time_mix_q, self.time_mix_k,
                                                            self.time_mix_v)]
         quant = R.shift_quantize(x, *sig)
         B, T, _ = x.shape
         outs = []
-        for (codes, scales), proj in zip(quant, (self.q_proj, self.k_proj, self.v_proj)):
+        for (codes, scales), proj in zip(quant, projs):
             proj._quantize_weight()
             y = w8a8_gemm_out(codes, scales, proj.weight_codes, proj.weight_scales,
                               bias=None if proj.bias is None else proj.bias.detach().float(),
@@ -153,5 +164,9 @@ class RosaMixer(nn.Module):
             B, T, S = q_full.shape
             sign, _ = R.match_packed(qb.reshape(B * S, -1), kb.reshape(B * S, -1),
                                      vb.reshape(B * S, -1), T)
+        half_or_float = (torch.float32, torch.bfloat16, torch.float16)
+        if (not torch.is_grad_enabled() and x.dtype in half_or_float
+                and self.payload.dtype in half_or_float and B <= 65535):
+            return self._out(R.hard_out(sign.reshape(B, S, T), self.payload, x.dtype), residual)
         out = self.payload[None, :, None] * sign.reshape(B, S, T).float()
         return self._out(out.permute(0, 2, 1).to(x.dtype), residual)
