@@ -486,6 +486,17 @@ int ksd_ks3_vjp_finalize(const float *partials, int64_t n_row_blocks, int64_t F,
  * i.e. torch.tanh on an fp16 tensor (reference ksdraft/kernels/ks3_int8.py:365-366).
  */
 /*
+ * K9 — a training forward's geometry from its fp32 masters (reference ksdraft/kernels/ks3_int8.py:
+ * 262-277, 158-165), in one launch: quantize_last_dim of the (F, 6) coefficient rows, of
+ * softplus(raw_scale) + 1e-4 and of tanh(raw_shift) / 2 (one value a row), and the latter two
+ * dequantized to fp16. Codes int8, scales and *16 fp16, each (F,) but spine_codes (F, 6).
+ */
+int ksd_ks3_pack_masters(const float *coefficients, const float *raw_scale, const float *raw_shift,
+                         int64_t F, int8_t *spine_codes, uint16_t *spine_scale, int8_t *scale_codes,
+                         uint16_t *scale_scales, int8_t *shift_codes, uint16_t *shift_scales,
+                         uint16_t *scale16, uint16_t *shift16, void *stream);
+
+/*
  * K11 — _grad_handoff (reference ksdraft/kernels/ks3_int8.py:75-84) on the device: out =
  * fp32(fp16(t)) when every fp16(t[i]) is finite, else t, decided by *flag (int32, zeroed by
  * the caller; set to 1 here when an element overflows fp16 or is NaN). t, out (n,) fp32;

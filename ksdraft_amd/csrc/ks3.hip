@@ -1055,6 +1055,37 @@ __global__ void ks3_tanh16_kernel(const uint16_t *__restrict__ x, int64_t n, uin
   y[i] = __builtin_bit_cast(uint16_t, tanh2(a, tab)[0]);
 }
 
+// A training forward's geometry from the fp32 masters (ks3_int8.py:262-277), one thread per chart: the
+// coefficient row's codes and scale, and the warp scalars' (softplus(raw) + 1e-4 and tanh(raw) / 2, with
+// torch's formulas and the same library functions, so the same bits) codes, scales and fp16 values. Eleven
+// launches of 4 to 5 us on 5888 values; this kernel is bound by its launch too: 55 us of
+// device time to 4.7, with the paired transposes about 20 us of the cell's 1220 at 8192 rows.
+__global__ __launch_bounds__(256) void ks3_pack_masters_kernel(
+    const float *__restrict__ coeff, const float *__restrict__ raw_scale, const float *__restrict__ raw_shift,
+    int64_t F, int8_t *__restrict__ spine_codes, uint16_t *__restrict__ spine_scale, int8_t *__restrict__ wsc,
+    uint16_t *__restrict__ wss, int8_t *__restrict__ whc, uint16_t *__restrict__ whs,
+    uint16_t *__restrict__ scale16, uint16_t *__restrict__ shift16) {
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c >= F) return;
+  float v[6];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) v[i] = coeff[c * 6 + i];
+  const float s = group_scale(abs_max<6>(v));
+  spine_scale[c] = scale_bits(s);
+#pragma unroll
+  for (int i = 0; i < 6; ++i) spine_codes[c * 6 + i] = code_of(v[i] / s);
+  const float a = raw_scale[c];
+  const float w[2] = {(a > 20.0f ? a : log1pf(expf(a))) + 1e-4f, 0.5f * tanhf(raw_shift[c])};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float ws = group_scale(fabsf(w[i]));
+    const int8_t q = code_of(w[i] / ws);
+    (i ? whc : wsc)[c] = q;
+    (i ? whs : wss)[c] = scale_bits(ws);
+    (i ? shift16 : scale16)[c] = f16_bits((float)q * ws);
+  }
+}
+
 // ---------------------------------------------------------------- launchers
 template <int G>
 static void launch_spine(bool vec, dim3 grid, hipStream_t st, const uint16_t *coords, int64_t M,
@@ -1670,4 +1701,19 @@ extern "C" int ksd_grad_handoff(const float *t, int64_t n, int *flag, float *out
     hipLaunchKernelGGL(handoff_select_kernel, dim3(grid), dim3(256), 0, st, t, n, (const int *)flag, out);
   }
   return check_launch("grad_handoff");
+}
+
+extern "C" int ksd_ks3_pack_masters(const float *coefficients, const float *raw_scale, const float *raw_shift,
+                                    int64_t F, int8_t *spine_codes, uint16_t *spine_scale, int8_t *scale_codes,
+                                    uint16_t *scale_scales, int8_t *shift_codes, uint16_t *shift_scales,
+                                    uint16_t *scale16, uint16_t *shift16, void *stream) {
+  if (F < 0 || F > (1LL << 31) / 1024) return fail(KSD_EINVAL, "ks3_pack_masters: F out of range");
+  if (F == 0) return KSD_OK;
+  if (!coefficients || !raw_scale || !raw_shift || !spine_codes || !spine_scale || !scale_codes || !scale_scales ||
+      !shift_codes || !shift_scales || !scale16 || !shift16)
+    return fail(KSD_EINVAL, "ks3_pack_masters: null pointer");
+  ks3_pack_masters_kernel<<<(unsigned)cdiv(F, 256), 256, 0, (hipStream_t)stream>>>(
+      coefficients, raw_scale, raw_shift, F, spine_codes, spine_scale, scale_codes, scale_scales, shift_codes,
+      shift_scales, scale16, shift16);
+  return check_launch("ks3_pack_masters");
 }

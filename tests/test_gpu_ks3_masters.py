@@ -1,0 +1,36 @@
+"""The KS3 geometry packed from its masters in one launch against its eleven calls, bit for bit:
+block remainders, both sides of softplus's threshold, zeros, large and subnormal values, infinities;
+and what keeps the calls."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from ksdraft_amd.kernels import ks3_int8 as ki
+from ksdraft_amd.kernels.quant import dequantize_last_dim, quantize_last_dim
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("Fn", [1, 255, 257, 100003])
+def test_masters_packed_in_one_launch(Fn):
+    g = torch.Generator().manual_seed(Fn)
+    co = torch.randn(Fn, 1, 6, generator=g) * 0.05
+    rs, rh = torch.randn(Fn, generator=g) * 12, torch.randn(Fn, generator=g) * 3
+    edge = torch.tensor([0.0, -0.0, 20.0, 20.000002, 19.999998, 88.0, -88.0, -104.0, 1e30, -1e30, 1e-30, 1e-40,
+                         float("inf"), -float("inf")])
+    n = min(Fn, len(edge))
+    rs[:n], rh[:n], co.view(Fn, 6)[:n, 0] = edge[:n], edge[:n], edge[:n]
+    co.view(Fn, 6)[n // 2] = 0.0
+    co, rs, rh = co.to(DEV), rs.to(DEV), rh.to(DEV)
+    got = ki.pack_masters(co, rs, rh)
+    sq, ss = ki.pack_spine(co)
+    wsc, wss = quantize_last_dim((F.softplus(rs) + 1e-4).reshape(-1, 1))
+    whc, whs = quantize_last_dim((0.5 * torch.tanh(rh)).reshape(-1, 1))
+    want = (sq, ss, wsc, wss, whc, whs, dequantize_last_dim(wsc, wss).reshape(-1).half(),
+            dequantize_last_dim(whc, whs).reshape(-1).half())
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+    assert ki.pack_masters(co.expand(Fn, 2, 6), rs, rh) is None  # rank 2
+    assert ki.pack_masters(co.half(), rs, rh) is None
