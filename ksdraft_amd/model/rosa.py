@@ -164,9 +164,10 @@ class RosaMixer(nn.Module):
             B, T, S = q_full.shape
             sign, _ = R.match_packed(qb.reshape(B * S, -1), kb.reshape(B * S, -1),
                                      vb.reshape(B * S, -1), T)
-        half_or_float = (torch.float32, torch.bfloat16, torch.float16)
-        if (not torch.is_grad_enabled() and x.dtype in half_or_float
-                and self.payload.dtype in half_or_float and B <= 65535):
+        from ..kernels.linear import Int8Linear
+        types = (torch.float32, torch.bfloat16, torch.float16)
+        if (not torch.is_grad_enabled() and isinstance(self.out_proj, Int8Linear) and x.dtype in types
+                and self.payload.dtype in types and B <= 65535):  # the products in one launch
             return self._out(R.hard_out(sign.reshape(B, S, T), self.payload, x.dtype), residual)
         out = self.payload[None, :, None] * sign.reshape(B, S, T).float()
         return self._out(out.permute(0, 2, 1).to(x.dtype), residual)
