@@ -258,6 +258,11 @@ def match_packed(q_bits: torch.Tensor, k_bits: torch.Tensor, v_bits: torch.Tenso
     return sign, mj
 
 
+def hard_out_fits(B: int, S: int) -> bool:
+    """The shapes hard_out takes: ksd_rosa_hard's grid holds B and S / 64 blocks in y and z."""
+    return B <= 65535 and S <= 64 * 65535
+
+
 def hard_out(sign: torch.Tensor, payload: torch.Tensor, out_dtype=torch.float32) -> torch.Tensor:
     """(B, S, T) int8 sign -> (B, T, S) payload[s] * sign (rosa_credit_gpu.py:75)."""
     dev = _lib.require_gpu(sign, payload)

@@ -167,7 +167,7 @@ class RosaMixer(nn.Module):
         from ..kernels.linear import Int8Linear
         types = (torch.float32, torch.bfloat16, torch.float16)
         if (not torch.is_grad_enabled() and isinstance(self.out_proj, Int8Linear) and x.dtype in types
-                and self.payload.dtype in types and B <= 65535):  # the products in one launch
+                and self.payload.dtype in types and R.hard_out_fits(B, S)):  # the products in one launch
             return self._out(R.hard_out(sign.reshape(B, S, T), self.payload, x.dtype), residual)
         out = self.payload[None, :, None] * sign.reshape(B, S, T).float()
         return self._out(out.permute(0, 2, 1).to(x.dtype), residual)
