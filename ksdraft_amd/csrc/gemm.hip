@@ -947,9 +947,11 @@ __global__ __launch_bounds__(256) void splitk_combine_kernel(const float *__rest
 // launch, 16 bytes per thread: a GEMM whose K is no multiple of 128 needs both of its
 // operands padded, a paired launch all four, which took a fill and a copy launch each. Bound by
 // the launch at these sizes (5 us for the four operands of a 509 x 1000 -> 777 linear's
-// backward), so one launch of 16-byte threads serves any number of rows. With the one-pass
+// backward), so one launch of 16-byte threads serves any number of rows; past kPadBlocks blocks
+// (16 GiB) the threads walk on, as a launch holds fewer than 2^32 of them. With the one-pass
 // ragged quantizers that linear's training pass went from 336 to 297 us, 20 launches to 8.
 constexpr int kPadMax = 4;
+constexpr int64_t kPadBlocks = 1 << 22;
 struct PadOperand {
   const int8_t *src;
   int8_t *dst;
@@ -960,31 +962,33 @@ struct PadArg {
   PadOperand o[kPadMax];
   int n;
 };
-__global__ __launch_bounds__(256) void pad_codes_kernel(const PadArg a) {
-  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void pad_codes_kernel(const PadArg a, int64_t total) {
+  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < total; c += (int64_t)gridDim.x * 256) {
+    int64_t i = c;
 #pragma unroll
-  for (int j = 0; j < kPadMax; ++j) {
-    if (j >= a.n) return;
-    const PadOperand &o = a.o[j];
-    if (i < o.chunks) {
-      const int per = o.Kp / 16;
-      const int64_t row = i / per;
-      const int k0 = (int)(i - row * per) * 16;
-      const int8_t *p = o.src + row * o.K + k0;
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (k0 + 16 <= o.K) {
-        __builtin_memcpy(&v, p, 16);  // rows of any alignment
-      } else {
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
+    for (int j = 0; j < kPadMax; ++j) {
+      if (j >= a.n) break;
+      const PadOperand &o = a.o[j];
+      if (i < o.chunks) {
+        const int per = o.Kp / 16;
+        const int64_t row = i / per;
+        const int k0 = (int)(i - row * per) * 16;
+        const int8_t *p = o.src + row * o.K + k0;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (k0 + 16 <= o.K) {
+          __builtin_memcpy(&v, p, 16);  // rows of any alignment
+        } else {
+          uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int b = 0; b < 16; ++b)
-          if (k0 + b < o.K) w[b >> 2] |= (uint32_t)(uint8_t)p[b] << (8 * (b & 3));
-        v = make_uint4(w[0], w[1], w[2], w[3]);
+          for (int b = 0; b < 16; ++b)
+            if (k0 + b < o.K) w[b >> 2] |= (uint32_t)(uint8_t)p[b] << (8 * (b & 3));
+          v = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+        *(uint4 *)(o.dst + row * o.Kp + k0) = v;
+        break;
       }
-      *(uint4 *)(o.dst + row * o.Kp + k0) = v;
-      return;
+      i -= o.chunks;
     }
-    i -= o.chunks;
   }
 }
 
@@ -1171,8 +1175,7 @@ extern "C" int ksd_pad_codes(const KsdPadOperand *list, int n, void *stream) {
     total += o.rows * (o.Kp / 16);
   }
   if (total == 0) return KSD_OK;
-  if (cdiv(total, 256) > 0x7fffffffLL) return fail(KSD_EINVAL, "pad_codes: operands too large");
-  pad_codes_kernel<<<dim3((unsigned)cdiv(total, 256)), dim3(256), 0, (hipStream_t)stream>>>(a);
+  pad_codes_kernel<<<dim3((unsigned)min(cdiv(total, 256), kPadBlocks)), dim3(256), 0, (hipStream_t)stream>>>(a, total);
   return check_launch("pad_codes");
 }
 

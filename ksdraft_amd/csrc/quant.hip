@@ -1094,7 +1094,8 @@ extern "C" int ksd_int8_linear(const void *x, int x_dtype, int64_t M, int64_t x_
                    ((uintptr_t)w_codes | (uintptr_t)x_codes) % 8 == 0;
   const int rtw = four_rows(N, K) ? 4 : 1, rtx = four_rows(M, K) ? 4 : 1;
   const int64_t nbw = cdiv(N, 4 * rtw), nbx = cdiv(M, 4 * rtx);
-  if (vec && M > 0 && N > 0 && nbw + nbx <= 0x7fffffffLL) {
+  // a launch holds fewer than 2^32 threads: the two operands of the largest calls take one each
+  if (vec && M > 0 && N > 0 && nbw + nbx < (1 << 24)) {
     const dim3 grid((unsigned)(nbw + nbx), (unsigned)cdiv(K, 512));
     hipStream_t st = (hipStream_t)stream;
 #define KSD_PAIR(DT, RW, RX)                                                                                       \
@@ -1115,7 +1116,7 @@ extern "C" int ksd_int8_linear(const void *x, int x_dtype, int64_t M, int64_t x_
 #undef KSD_PAIR
     const int rc = check_launch("int8_linear");
     if (rc) return rc;
-  } else {  // unaligned rows: a launch each
+  } else {  // unaligned rows, or too many for one grid: a launch each
     int rc = ksd_quantize_lastdim(w, KSD_F32, N, K, K, 128, w_codes, w_scales, nullptr, 0.0f, stream);
     if (!rc) rc = ksd_quantize_lastdim(x, x_dtype, M, K, x_stride, 128, x_codes, x_scales, nullptr, 0.0f, stream);
     if (rc) return rc;
