@@ -269,7 +269,7 @@ extern "C" int ksd_transfer_cos(const float *f, const float *e_hat, int64_t M, i
   if (M < 0 || d < 0) return fail(KSD_EINVAL, "transfer_cos: negative shape");
   if (M == 0 || d == 0) return KSD_OK;
   if (!f || !e_hat || !cos_out || !norm_out) return fail(KSD_EINVAL, "transfer_cos: null pointer");
-  if (M > 0x7ffffff0LL || d > 0x7fffffffLL) return fail(KSD_EINVAL, "transfer_cos: too large");
+  if (!grid_fits(cdiv(M, 4), 256) || d > 0x7fffffffLL) return fail(KSD_EINVAL, "transfer_cos: too large");
   const bool vec = d % 4 == 0 && ((uintptr_t)f % 16) == 0 && ((uintptr_t)e_hat % 16) == 0;
   const dim3 grid((unsigned)cdiv(M, 4));
   hipStream_t st = (hipStream_t)stream;
@@ -287,7 +287,7 @@ extern "C" int ksd_transfer_grad(const float *f, const float *e_hat, const float
   if (M == 0 || d == 0) return KSD_OK;
   if (!f || !e_hat || !cos_in || !norm_in || !coef || !df || !grad_e)
     return fail(KSD_EINVAL, "transfer_grad: null pointer");
-  if (M > 0x7ffffff0LL || d > 0x7fffffffLL) return fail(KSD_EINVAL, "transfer_grad: too large");
+  if (!grid_fits(cdiv(M, 4), 256) || d > 0x7fffffffLL) return fail(KSD_EINVAL, "transfer_grad: too large");
   const bool vec = d % 4 == 0 && ((uintptr_t)f % 16) == 0 && ((uintptr_t)e_hat % 16) == 0 &&
                    ((uintptr_t)df % 16) == 0 && ((uintptr_t)grad_e % 16) == 0;
   const dim3 grid((unsigned)cdiv(M, 4));

@@ -1592,7 +1592,7 @@ extern "C" int ksd_ks3_spine_float(const void *x, int x_dtype, int64_t M, int64_
     return fail(KSD_EINVAL, "ks3_spine_float: h_codes and h_scales go together");
   if (!h && !h_codes) return fail(KSD_EINVAL, "ks3_spine_float: no output requested");
   if (M == 0 || F == 0) return KSD_OK;
-  if (F > (1LL << 28) || M > 0x7fffffffLL - kSpineFloatRows)
+  if (F > (1LL << 28) || M > 0x7fffffffLL - kSpineFloatRows || !grid_fits(cdiv(M, kSpineFloatRows), 256))
     return fail(KSD_EINVAL, "ks3_spine_float: too large");
   const size_t esz = x_dtype == KSD_F32 ? 4 : 2;
   const bool vec = (F & 7) == 0 && ((uintptr_t)x % 16) == 0 && (F * esz) % 16 == 0 &&

@@ -40,6 +40,10 @@ inline bool valid_group(int g) { return g == 32 || g == 64 || g == 128; }
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// A launch holds fewer than 2^32 threads along x: more wrap around, and the blocks past them
+// never run, without an error.
+inline bool grid_fits(int64_t blocks, int64_t threads) { return blocks <= 0xffffffffLL / threads; }
+
 // The device's CU count (persistent launches size their grids by it), cached per device.
 static inline int cu_count() {
   static int cached[64];

@@ -891,7 +891,7 @@ static int launch_quant_T(const void *x, const uint16_t *in_scales, int64_t nsc_
                           hipStream_t st) {
   const int64_t nbc = cdiv(C, 64), ngr = cdiv(R, group);
   const int64_t blocks = nbc * ngr;
-  if (blocks > 0x7fffffffLL) return fail(KSD_EINVAL, "quantize_transpose: tensor too large");
+  if (!grid_fits(blocks, 256)) return fail(KSD_EINVAL, "quantize_transpose: tensor too large");
   const dim3 g((unsigned)blocks), b(256);
   // 16-byte vector loads need an aligned base and a row pitch that is a multiple of 16 B
   const int esz = SRC == SRC_F32 ? 4 : SRC == SRC_I8 ? 1 : 2;
@@ -1066,12 +1066,13 @@ extern "C" int ksd_quantize_lastdim(const void *x, int x_dtype, int64_t rows, in
   if (!valid_group(group)) return fail(KSD_EINVAL, "group must be 32, 64 or 128, got %d", group);
   if (rows < 0 || K < 0 || x_stride < K) return fail(KSD_EINVAL, "bad quantize shape");
   if (rows == 0 || K == 0) return KSD_OK;
-  if (cdiv(rows * cdiv(K, group) * (group / 8), 256) > 0x7fffffffLL)
-    return fail(KSD_EINVAL, "quantize: tensor too large");
   hipStream_t st = (hipStream_t)stream;
   const int esz = x_dtype == KSD_F32 ? 4 : 2;
   const bool vec = (((uintptr_t)x) % 16 == 0) && ((x_stride * esz) % 16 == 0) &&
                    (K % 8 == 0) && (((uintptr_t)codes) % 8 == 0);
+  if (!grid_fits(vec && noise == nullptr && K <= (1 << 24) ? cdiv(rows, four_rows(rows, K) ? 16 : 4)
+                                                           : cdiv(rows * cdiv(K, group) * (group / 8), 256), 256))
+    return fail(KSD_EINVAL, "quantize: tensor too large");
   switch (x_dtype) {
     case KSD_F32: launch_rows_g<KSD_F32>(group, x, rows, K, x_stride, codes, scales, noise, dither2, vec, st); break;
     case KSD_BF16: launch_rows_g<KSD_BF16>(group, x, rows, K, x_stride, codes, scales, noise, dither2, vec, st); break;
@@ -1094,8 +1095,7 @@ extern "C" int ksd_int8_linear(const void *x, int x_dtype, int64_t M, int64_t x_
                    ((uintptr_t)w_codes | (uintptr_t)x_codes) % 8 == 0;
   const int rtw = four_rows(N, K) ? 4 : 1, rtx = four_rows(M, K) ? 4 : 1;
   const int64_t nbw = cdiv(N, 4 * rtw), nbx = cdiv(M, 4 * rtx);
-  // a launch holds fewer than 2^32 threads: the two operands of the largest calls take one each
-  if (vec && M > 0 && N > 0 && nbw + nbx < (1 << 24)) {
+  if (vec && M > 0 && N > 0 && grid_fits(nbw + nbx, 256)) {
     const dim3 grid((unsigned)(nbw + nbx), (unsigned)cdiv(K, 512));
     hipStream_t st = (hipStream_t)stream;
 #define KSD_PAIR(DT, RW, RX)                                                                                       \
@@ -1246,7 +1246,7 @@ extern "C" int ksd_embedding_gather_int8(const int8_t *codes, const uint16_t *sc
   if (n == 0 || d == 0) return KSD_OK;
   if (V == 0) return fail(KSD_EINVAL, "embedding_gather: empty table");
   if (!codes || !scales || !ids || !out) return fail(KSD_EINVAL, "embedding_gather: null pointer");
-  if (cdiv(n, 4) > 0x7fffffffLL) return fail(KSD_EINVAL, "embedding_gather: too many rows");
+  if (!grid_fits(cdiv(n, 4), 256)) return fail(KSD_EINVAL, "embedding_gather: too many rows");
   const int64_t nsc = cdiv(d, group);
   const bool vec = d % 8 == 0 && ((uintptr_t)codes & 7) == 0;
   const dim3 g((unsigned)cdiv(n, 4)), b(256);
@@ -1270,7 +1270,7 @@ extern "C" int ksd_dequantize_lastdim(const int8_t *codes, const uint16_t *scale
   if (group <= 0) return fail(KSD_EINVAL, "dequantize: group must be positive");
   if (rows == 0 || K == 0) return KSD_OK;
   const int64_t n = rows * K;
-  if (cdiv(n, 256) > 0x7fffffffLL) return fail(KSD_EINVAL, "dequantize: tensor too large");
+  if (!grid_fits(cdiv(n, 256), 256)) return fail(KSD_EINVAL, "dequantize: tensor too large");
   dequant_rows_kernel<<<(unsigned)cdiv(n, 256), 256, 0, (hipStream_t)stream>>>(
       codes, scales, rows, K, n_scales, group, out);
   return check_launch("dequantize_lastdim");
@@ -1362,7 +1362,7 @@ extern "C" int ksd_quantize_dual2(const void *x0, int64_t R0, int64_t C0, int8_t
   };
   const bool vec = vec16(x0, C0, codes0) && vec16(x1, C1, codes1);
   if (!fast(R0, C0) || !fast(R1, C1) ||
-      cdiv(C0, 128) * cdiv(R0, 128) + cdiv(C1, 128) * cdiv(R1, 128) > 0x7fffffffLL) {
+      !grid_fits(cdiv(C0, 128) * cdiv(R0, 128) + cdiv(C1, 128) * cdiv(R1, 128), 512)) {
     int rc = ksd_quantize_dual(x0, x_dtype, R0, C0, group, 1, codes0, scales0, codes_t0, scales_t0, stream);
     if (rc) return rc;
     return ksd_quantize_dual(x1, x_dtype, R1, C1, group, 1, codes1, scales1, codes_t1, scales_t1, stream);
@@ -1431,7 +1431,7 @@ extern "C" int ksd_ce_row_stats(const float *logits, int64_t R, int64_t C, const
   if (C == 0) return fail(KSD_EINVAL, "ce_row_stats: no classes");
   if (!logits || !targets || !row_max || !row_inv_sum || !row_loss)
     return fail(KSD_EINVAL, "ce_row_stats: null pointer");
-  if (R > 0x7fffffffLL) return fail(KSD_EINVAL, "ce_row_stats: too many rows");
+  if (!grid_fits(R, 256)) return fail(KSD_EINVAL, "ce_row_stats: too many rows");
   hipStream_t st = (hipStream_t)stream;
   const bool vec = C % 16 == 0 && ((uintptr_t)logits) % 16 == 0;
   if (vec)
@@ -1470,7 +1470,7 @@ extern "C" int ksd_ce_backward_quant_dual(const float *logits, int64_t R, int64_
   }
   // tensors past the tile kernel's 32-bit offsets: dY into dy_out (required here), then the dual quantizer on it
   if (!dy_out) return fail(KSD_EINVAL, "ce_backward_quant_dual: this shape needs dy_out (R x C fp32)");
-  if (cdiv(R * C, 256) > 0x7fffffffLL) return fail(KSD_EINVAL, "ce_backward_quant_dual: tensor too large");
+  if (!grid_fits(cdiv(R * C, 256), 256)) return fail(KSD_EINVAL, "ce_backward_quant_dual: tensor too large");
   ce_dy_kernel<<<(unsigned)cdiv(R * C, 256), 256, 0, st>>>(logits, R, C, ce);
   const int rc = check_launch("ce_backward_quant_dual (dY)");
   if (rc) return rc;
@@ -1490,7 +1490,7 @@ extern "C" int ksd_adamw_requant(float *param, const float *grad, float *exp_avg
     return fail(KSD_EINVAL, "adamw_requant: codes and scales go together");
   const int64_t ng = cdiv(K, 128);
   const int64_t blocks = cdiv(rows * ng, 16);
-  if (blocks > 0x7fffffffLL) return fail(KSD_EINVAL, "adamw_requant: tensor too large");
+  if (!grid_fits(blocks, 256)) return fail(KSD_EINVAL, "adamw_requant: tensor too large");
   const AdamArgs a{decay, one_minus_beta1, beta2, one_minus_beta2, eps, step_size, bias_correction2_sqrt};
   auto al = [](const void *q, uintptr_t n) { return ((uintptr_t)q) % n == 0; };
   const bool vec = K % 8 == 0 && al(param, 16) && al(grad, 16) && al(exp_avg, 16) && al(exp_avg_sq, 16) &&
@@ -1519,7 +1519,7 @@ extern "C" int ksd_adamw_requant_multi(const KsdAdamTensor *tensors, int n, cons
       return fail(KSD_EINVAL, "adamw_requant_multi: tensor %d: null pointer", i);
     if ((t.codes == nullptr) != (t.scales == nullptr))
       return fail(KSD_EINVAL, "adamw_requant_multi: tensor %d: codes and scales go together", i);
-    if (cdiv(t.rows * cdiv(t.K, 128), 16) > 0x3fffffffLL)
+    if (!grid_fits(cdiv(t.rows * cdiv(t.K, 128), 16), 256))
       return fail(KSD_EINVAL, "adamw_requant_multi: tensor %d too large", i);
   }
   hipStream_t st = (hipStream_t)stream;
@@ -1538,7 +1538,7 @@ extern "C" int ksd_adamw_requant_multi(const KsdAdamTensor *tensors, int n, cons
     const KsdAdamTensor &t = tensors[i];
     if (t.rows == 0 || t.K == 0) continue;
     const int64_t ng = cdiv(t.K, 128), nb = cdiv(t.rows * ng, 16);
-    if (b.n == kAdamBatch || blocks + nb > 0x7fffffffLL) {
+    if (b.n == kAdamBatch || !grid_fits(blocks + nb, 256)) {
       const int rc = flush();
       if (rc) return rc;
     }
@@ -1564,7 +1564,7 @@ extern "C" int ksd_requant_transpose_multi(const KsdRequantT *list, int n, int g
     if (t.R == 0 || t.C == 0) continue;
     if (!t.codes || !t.scales || !t.codes_t || !t.scales_t)
       return fail(KSD_EINVAL, "requant_transpose_multi: entry %d: null pointer", i);
-    if (cdiv(t.C, 64) * cdiv(t.R, 128) > 0x3fffffffLL)
+    if (!grid_fits(cdiv(t.C, 64) * cdiv(t.R, 128), 256))
       return fail(KSD_EINVAL, "requant_transpose_multi: entry %d too large", i);
   }
   hipStream_t st = (hipStream_t)stream;
@@ -1582,7 +1582,7 @@ extern "C" int ksd_requant_transpose_multi(const KsdRequantT *list, int n, int g
     const KsdRequantT &t = list[i];
     if (t.R == 0 || t.C == 0) continue;
     const int64_t nbc = cdiv(t.C, 64), ngr = cdiv(t.R, 128), nb = nbc * ngr;
-    if (b.n == kRqtBatch || blocks + nb > 0x7fffffffLL) {
+    if (b.n == kRqtBatch || !grid_fits(blocks + nb, 256)) {
       const int rc = flush();
       if (rc) return rc;
     }
@@ -1606,7 +1606,6 @@ extern "C" int ksd_layernorm_quant(const void *x, int x_dtype, int64_t rows, int
   if (!(eps >= 0.0f) || eps > 1.0f) return fail(KSD_EINVAL, "layernorm_quant: eps must be in [0, 1]");
   if (rows == 0) return KSD_OK;
   if (!x || !codes || !scales) return fail(KSD_EINVAL, "layernorm_quant: null pointer");
-  if (rows > 0x7fffffffLL) return fail(KSD_EINVAL, "layernorm_quant: too many rows");
   hipStream_t st = (hipStream_t)stream;
   const int esz = x_dtype == KSD_F32 ? 4 : 2;
   const bool vec = (((uintptr_t)x) % 16 == 0) && ((x_stride * esz) % 16 == 0) && (d % 8 == 0) &&
@@ -1614,6 +1613,7 @@ extern "C" int ksd_layernorm_quant(const void *x, int x_dtype, int64_t rows, int
   const bool v = vec && (((uintptr_t)weight) % 16 == 0) && (((uintptr_t)bias) % 16 == 0);
   const int ng = (int)cdiv(d, 128);
   const int threads = (int)cdiv(cdiv(d, 8), 64) * 64;
+  if (!grid_fits(rows, threads)) return fail(KSD_EINVAL, "layernorm_quant: too many rows");
   const dim3 grid((unsigned)rows);
 #define KSD_LN(DT, V) \
   ln_quant_kernel<DT, V><<<grid, threads, 0, st>>>(x, rows, (int)d, x_stride, weight, bias, eps, ng, codes, scales, y_out, mean_out, rstd_out)

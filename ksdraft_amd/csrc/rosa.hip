@@ -685,7 +685,7 @@ extern "C" int ksd_rosa_shift_quant(const void *x, int x_dtype, int64_t B, int64
       !v_codes || !v_scales)
     return fail(KSD_EINVAL, "rosa_shift_quant: null pointer");
   const int64_t ng = cdiv(d, group);
-  if (rows > 0x7fffffff - 64 || d > (1 << 28) || T > 0x7fffffff)
+  if (rows > 0x7fffffff - 64 || !grid_fits(cdiv(rows, 16), 256) || d > (1 << 28) || T > 0x7fffffff)
     return fail(KSD_EINVAL, "rosa_shift_quant: too large");
   const size_t esz = x_dtype == KSD_F32 ? 4 : 2;
   auto al = [](const void *p, size_t a) { return ((uintptr_t)p % a) == 0; };
@@ -850,7 +850,7 @@ extern "C" int ksd_rosa_match(const uint32_t *q_bits, const uint32_t *k_bits, co
   if (n_streams > 0x7fffffff) return fail(KSD_EINVAL, "rosa_match: too many streams");
   const int W = (int)cdiv(T, 32);
   const int nchunks = (int)cdiv(T, kMatchChunk);
-  if (n_streams * nchunks > 0x7fffffffLL) return fail(KSD_EINVAL, "rosa_match: too many streams");
+  if (!grid_fits(n_streams * nchunks, kMatchChunk)) return fail(KSD_EINVAL, "rosa_match: too many streams");
   hipLaunchKernelGGL(rosa_match_kernel, dim3((unsigned)(n_streams * nchunks)), dim3(kMatchChunk),
                      3 * W * sizeof(uint32_t), (hipStream_t)stream, q_bits, k_bits, v_bits, (int)T, W,
                      lmax, (int)n_streams, nchunks, sign, match_j);
@@ -1993,7 +1993,7 @@ extern "C" int ksd_rosa_credits(const uint32_t *q_bits, const uint32_t *k_bits, 
   const int W = (int)cdiv(T, 32);
   const size_t lds = (4 + 3 * (size_t)W + kCredWaves * (size_t)kCredWave32) * sizeof(uint32_t);
   if (lds > 64 * 1024) return fail(KSD_EINVAL, "rosa_credits: T too large for LDS");
-  if (B * S > 0x7fffffff || B * S * cdiv(T, kCredChunk) > 0x7fffffff)
+  if (!grid_fits(B * S, 256) || B * S * cdiv(T, kCredChunk) > 0x7fffffff)
     return fail(KSD_EINVAL, "rosa_credits: too many streams");
   hipStream_t st = (hipStream_t)stream;
   unsigned long long *sums = (unsigned long long *)credit_sums;

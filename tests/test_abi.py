@@ -107,6 +107,28 @@ def test_ks3_validation_paths_without_gpu():
                                      p, p, a, None) == 0  # empty: nothing to launch
 
 
+def test_launches_of_2_to_the_32_threads_are_refused():
+    """Validation only: such a launch would wrap around and leave rows unwritten."""
+    lib = _lib.load()
+    p = ctypes.c_void_p(256)  # never dereferenced
+    rows = 1 << 28
+    calls = {
+        "quantize": lambda: lib.ksd_quantize_lastdim(p, 0, rows, 128, 128, 128, p, p, None, 0.0, None),
+        "quantize, narrow": lambda: lib.ksd_quantize_lastdim(p, 0, rows, 1, 1, 128, p, p, None, 0.0, None),
+        "dequantize": lambda: lib.ksd_dequantize_lastdim(p, p, 1 << 16, 1 << 16, 512, 128, p, None),
+        "embedding": lambda: lib.ksd_embedding_gather_int8(p, p, p, 1 << 26, 8, 8, 128, p, 0, None),
+        "row statistics": lambda: lib.ksd_ce_row_stats(p, 1 << 24, 8, p, -100, p, p, p, None),
+        "layer norm": lambda: lib.ksd_layernorm_quant(p, 0, 1 << 26, 8, 8, p, p, 1e-5, 128, p, p, None, None,
+                                                      None, None),
+        "match": lambda: lib.ksd_rosa_match(p, p, p, 1 << 24, 8, 7, p, None, None),
+        "credits": lambda: lib.ksd_rosa_credits(p, p, p, p, p, p, 1, 8, 1 << 24, 7, p, p, p, None),
+    }
+    for name, f in calls.items():
+        assert f() == 1, name
+        lib.ksd_last_error(buf := ctypes.create_string_buffer(256), 256)
+        assert b"too large" in buf.value or b"too many" in buf.value, (name, buf.value)
+
+
 def test_single_hip_runtime_in_process():
     _lib.load()
     maps = open("/proc/self/maps").read()
