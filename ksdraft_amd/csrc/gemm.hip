@@ -1140,6 +1140,17 @@ static int gemm_checks(const int8_t *a, const int8_t *w, int64_t M, int64_t N, i
   return KSD_OK;
 }
 
+// The group-128 kernel addresses an operand's 128-row tile and the 32 output rows of a sub-tile
+// from one base with 32-bit offsets: reads past 2^31 bytes would leave the operand, and store
+// offsets past 2^32 (2^31 where the last tile masks columns) would come round into valid rows.
+static int gemm_offsets_check(int64_t M, int64_t N, int64_t K, int dtype) {
+  const int64_t rows = min(max(M, N), (int64_t)BM) - 1, slab = 32 * N * (dtype == KSD_F32 ? 4 : 2);
+  if (rows * K + BK > 1LL << 31 || slab >= 1LL << 32 || (slab > 1LL << 31 && N % BN != 0))
+    return fail(KSD_EINVAL, "w8a8_gemm: M=%lld, N=%lld, K=%lld exceed the kernel's 32-bit tile offsets",
+                (long long)M, (long long)N, (long long)K);
+  return KSD_OK;
+}
+
 }  // namespace ksd
 
 using namespace ksd;
@@ -1151,6 +1162,7 @@ extern "C" int ksd_w8a8_gemm_nt(const int8_t *a, const uint16_t *a_scales, const
   int rc = gemm_checks(a, w, M, N, K, group);
   if (rc != KSD_OK) return rc;
   if (M == 0 || N == 0 || K == 0) return KSD_OK;
+  if (group == 128 && (rc = gemm_offsets_check(M, N, K, y_dtype))) return rc;
   hipStream_t st = (hipStream_t)stream;
   switch (group) {
     case 32: return launch_o<32>(a, a_scales, w, w_scales, (int)M, (int)N, (int)K, bias, y, y_dtype, st);
@@ -1201,6 +1213,7 @@ extern "C" int ksd_w8a8_gemm_nt_ex(const int8_t *a, const uint16_t *a_scales, co
   }
   if (M == 0 || N == 0) return KSD_OK;
   if (K == 0) return fail(KSD_EINVAL, "w8a8_gemm_nt_ex: K = 0 (the host wrapper handles it)");
+  if (group == 128 && (rc = gemm_offsets_check(M, N, K, y_dtype))) return rc;
   const int splits = group == 128 ? g128_splits(M, N, K) : 1;
   hipStream_t st = (hipStream_t)stream;
   if (splits > 1) {
@@ -1244,6 +1257,7 @@ extern "C" int ksd_w8a8_gemm_pair(const int8_t *a0, const uint16_t *a0_scales, c
       return fail(KSD_ETYPE, "w8a8_gemm_pair: output dtype %d (fp32, bf16 or fp16 only)", dt[i]);
     if (M[i] > 0 && N[i] > 0 && K[i] == 0)
       return fail(KSD_EINVAL, "w8a8_gemm_pair: K = 0 (the host wrapper handles it)");
+    if (M[i] > 0 && N[i] > 0 && (rc = gemm_offsets_check(M[i], N[i], K[i], dt[i]))) return rc;
   }
   const bool e0 = M0 == 0 || N0 == 0, e1 = M1 == 0 || N1 == 0;
   hipStream_t st = (hipStream_t)stream;
@@ -1277,6 +1291,7 @@ extern "C" int ksd_ks3_project_fused(const int8_t *a, const uint16_t *a_scales, 
   if (F > (1LL << 31) / BM) return fail(KSD_EINVAL, "ks3_project_fused: F too large");
   if (M == 0 || F == 0) return KSD_OK;
   if (K == 0) return fail(KSD_EINVAL, "ks3_project_fused: K = 0 (the host wrapper handles it)");
+  if ((rc = gemm_offsets_check(M, F, K, KSD_F32))) return rc;
   hipStream_t st = (hipStream_t)stream;
   // Few rows: the accumulator fits where the table would lie (256 values a chart), and the GEMM followed by
   // the table-free spine is the faster form (us, this after the single launch: 16 x 1536 -> 5888 27.2, 9.4;

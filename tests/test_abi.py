@@ -129,6 +129,22 @@ def test_launches_of_2_to_the_32_threads_are_refused():
         assert b"too large" in buf.value or b"too many" in buf.value, (name, buf.value)
 
 
+def test_gemm_shapes_past_its_tile_offsets_are_refused():
+    """Validation only: reads would leave the operands, stores would land in other rows."""
+    lib = _lib.load()
+    p = ctypes.c_void_p(256)  # never dereferenced
+    for M, N, K, dt in ((200, 8, 17039360, 0), (8, 200, 17039360, 1),
+                        (1, (1 << 24) + 1, 128, 0), (1, 1 << 25, 128, 0), (40, (1 << 25) + 5, 128, 1)):
+        assert lib.ksd_w8a8_gemm_nt(p, p, p, p, M, N, K, 128, None, p, dt, None) == 1, (M, N, K)
+        assert lib.ksd_w8a8_gemm_nt_ex(p, p, p, p, M, N, K, 128, None, None, p, dt, p, 1 << 40, None) == 1
+        assert lib.ksd_w8a8_gemm_pair(p, p, p, p, 4, 4, 128, p, 0, p, p, p, p, M, N, K, p, dt, p, 1 << 40,
+                                      None) == 1
+        lib.ksd_last_error(buf := ctypes.create_string_buffer(256), 256)
+        assert b"offsets" in buf.value
+    # an empty product has no offsets
+    assert lib.ksd_w8a8_gemm_nt(p, p, p, p, 0, 200, 1 << 25, 128, None, p, 0, None) == 0
+
+
 def test_single_hip_runtime_in_process():
     _lib.load()
     maps = open("/proc/self/maps").read()
