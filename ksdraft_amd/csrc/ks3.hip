@@ -505,12 +505,12 @@ __global__ void __launch_bounds__(kSpineThreads) ks3_spine_fused_kernel(
   }
 }
 
-// Either spine on few rows (M F up to kDirectValues): the same values without the table, whose kernel
-// evaluates 256 indices of every chart and whose readers first copy 64 or 128 KB of it into LDS. Block =
-// 8 rows x 32 lanes of a 128-chart segment; a lane evaluates its row's 4 increments itself, about 80
-// VALU instructions each (six divisions by 127), so its time grows with M F where the table's reader
-// takes 30 us at least. Measured (us, the fused contract, table and reader -> this kernel): 16 x 5888
-// 39.8 -> 3.8, 256 x 5888 37.4 -> 8.8, 1024 x 5888 36.1 -> 26.2, 3001 x 256 30.6 -> 5.8.
+// Either spine on few rows (spine_direct): the same values without the table, whose kernel evaluates 256
+// indices of every chart and whose readers first copy 64 or 128 KB of it into LDS. Block = 8 rows x 32 lanes
+// of a 128-chart segment; a lane evaluates its row's 4 increments itself, about 80 VALU instructions each (six
+// divisions by 127), so its time grows with M F, 3.7 us (fused) and 4.1 us (composed) a million values.
+// Measured (us, the fused contract, 512-row table readers -> this kernel): 16 x 5888 36.3 -> 4.6, 500 x 2944
+// 34.0 -> 9.6, 1024 x 5888 37.6 -> 26.7.
 template <bool FUSED, int G, bool VEC>
 __global__ void __launch_bounds__(256) ks3_spine_rows_kernel(
     const void *__restrict__ in, int64_t M, int64_t F, const int8_t *__restrict__ spine_codes,
@@ -1109,10 +1109,17 @@ static void launch_fused(bool vec, dim3 grid, hipStream_t st, const float *acc, 
                        M, F, table, hq, hs, ng, rpb);
 }
 
-// Where the table-free kernel is the faster one: at 1024 x 5888 (6.0e6 values) 26.2 against 36.1 us, at
-// 3001 x 2944 (8.8e6) 37.3 against 33.9.
-constexpr int64_t kDirectValues = 7 << 20;
-static bool spine_direct(int64_t M, int64_t F) { return M <= 8 * 65535 && M <= kDirectValues / F; }
+// Where the table-free kernel is the faster one. Its time goes with M and the charts of whole segments; the
+// table costs as much as some hundred rows of every chart, and its launch and copies as much as a few million
+// values; element loads (F % 4 != 0) slow its reader more. Both sides (us, table-free and table): composed
+// 1464 x 1024 10.7, 11.1; 2441 x 1024 14.8, 14.4; 28125 x 256 34.3, 19.0; 424 x 5888 15.1, 20.3; 849 x 5888
+// 25.7, 24.2; 2049 x 2049 23.7, 27.5; 4504 x 777 22.0, 19.9. Fused 3417 x 1024 16.8, 16.6; 5859 x 1024 25.1,
+// 19.6; 1019 x 5888 25.6, 28.9; 1222 x 5888 30.2, 28.9; 240 x 30000 32.3, 45.7.
+static bool spine_direct(bool fused, int64_t M, int64_t F) {
+  const int64_t cols = cdiv(F, 128) * 128;
+  const int64_t rows = fused || F % 4 ? 600 + 3400000 / cols : 460 + 1200000 / cols;
+  return M <= min(rows, (int64_t)(8 * 65535));
+}
 
 template <bool FUSED, int G>
 static void launch_rows(bool vec, hipStream_t st, const void *in, int64_t M, int64_t F,
@@ -1423,8 +1430,7 @@ __global__ __launch_bounds__(256) void handoff_fixup_kernel(const float *__restr
 
 using namespace ksd;
 
-// The fused contract's per-chart increment table (F x 256 fp32), for the fused projection
-// GEMM in gemm.hip.
+// The fused contract's spine on an accumulator of few rows, for the fused projection in gemm.hip.
 int ksd::ks3_fused_rows(const float *acc, int64_t M, int64_t F, const int8_t *spine_codes,
                         const uint16_t *spine_scale, const uint16_t *warp_scale, const uint16_t *warp_shift,
                         const int8_t *tanh_lut, int group, int8_t *h_codes, uint16_t *h_scales, hipStream_t st) {
@@ -1433,6 +1439,8 @@ int ksd::ks3_fused_rows(const float *acc, int64_t M, int64_t F, const int8_t *sp
                              tanh_lut, nullptr, h_codes, h_scales);
 }
 
+// The fused contract's per-chart increment table (F x 256 fp32), for the fused projection
+// GEMM in gemm.hip.
 int ksd::ks3_fused_table(const int8_t *spine_codes, const uint16_t *spine_scale,
                          const uint16_t *warp_scale, const uint16_t *warp_shift, const int8_t *tanh_lut,
                          int64_t F, float *table, hipStream_t st) {
@@ -1474,7 +1482,7 @@ extern "C" int ksd_ks3_spine_fwd(const uint16_t *coords, int64_t M, int64_t F,
                    ((uintptr_t)h_codes & 3) == 0;
   const int64_t ng = cdiv(F, group);
   hipStream_t st = (hipStream_t)stream;
-  if (spine_direct(M, F))
+  if (spine_direct(false, M, F))
     return launch_rows_g<false>(group, vec, st, coords, M, F, spine_codes, spine_scale, warp_scale, warp_shift,
                                 tanh_lut, h, h_codes, h_scales);
   const int rpb = spine_rows_per_block(false, M, F);
@@ -1559,7 +1567,7 @@ extern "C" int ksd_ks3_spine_fused(const float *acc, int64_t M, int64_t F,
   const bool vec = (F & 3) == 0 && ((uintptr_t)acc & 15) == 0 && ((uintptr_t)h_codes & 3) == 0;
   const int64_t ng = cdiv(F, group);
   hipStream_t st = (hipStream_t)stream;
-  if (spine_direct(M, F))
+  if (spine_direct(true, M, F))
     return ks3_fused_rows(acc, M, F, spine_codes, spine_scale, warp_scale, warp_shift, tanh_lut, group,
                           h_codes, h_scales, st);
   const int rpb = spine_rows_per_block(true, M, F);
@@ -1615,6 +1623,12 @@ extern "C" int ksd_ks3_spine_float(const void *x, int x_dtype, int64_t M, int64_
 #undef KSD_SF_G
 #undef KSD_SFA
   return check_launch("ks3_spine_float");
+}
+
+extern "C" int ksd_ks3_spine_needs_table(int64_t M, int64_t F, int fused, int *needed) {
+  if (M < 0 || F < 0 || !needed) return fail(KSD_EINVAL, "ks3_spine_needs_table: bad arguments");
+  *needed = M > 0 && F > 0 && !spine_direct(fused != 0, M, F);
+  return KSD_OK;
 }
 
 extern "C" int ksd_ks3_vjp_row_blocks(int64_t M, int64_t *n_row_blocks) {
