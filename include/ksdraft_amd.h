@@ -297,6 +297,12 @@ int ksd_w8a8_gemm_nt(const int8_t *a, const uint16_t *a_scales, const int8_t *w,
 int ksd_w8a8_gemm_splits(int64_t M, int64_t N, int64_t K, int group, int *splits);
 
 /*
+ * Whether the group-128 GEMM of this shape runs in the kernel for few rows (1; no pair, and the
+ * K-part workspace then stays untouched) or in the persistent one (0). The outputs are the same.
+ */
+int ksd_w8a8_gemm_few_rows(int64_t M, int64_t N, int64_t K, int *few_rows);
+
+/*
  * The zero padding of a GEMM's code operands along K (reference ksdraft/kernels/gemm.py:71-73),
  * up to four operands in one launch: dst (rows, Kp) = src (rows, K) with Kp - K zeros per row.
  *   Kp a multiple of 16, Kp >= K; dst 16-byte aligned, src rows of any alignment; n <= 4

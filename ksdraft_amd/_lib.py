@@ -32,6 +32,7 @@ SIGNATURES = {
     "ksd_last_error": [ctypes.c_char_p, ctypes.c_size_t],
     "ksd_quantize_lastdim": [_P, _INT, _I64, _I64, _I64, _INT, _P, _P, _P, _F, _P],
     "ksd_int8_linear": [_P, _INT, _I64, _I64, _P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _INT, _P, _I64, _P],
+    "ksd_w8a8_gemm_few_rows": [_I64, _I64, _I64, _P],
     "ksd_ks3_spine_needs_table": [_I64, _I64, _INT, _P],
     "ksd_ks3_pack_masters": [_P, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P],
     "ksd_rosa_projections": [_P, _INT, _I64, _I64, _I64, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _P],

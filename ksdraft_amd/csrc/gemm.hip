@@ -1200,6 +1200,14 @@ extern "C" int ksd_w8a8_gemm_splits(int64_t M, int64_t N, int64_t K, int group, 
   return KSD_OK;
 }
 
+extern "C" int ksd_w8a8_gemm_few_rows(int64_t M, int64_t N, int64_t K, int *few_rows) {
+  int rc = gemm_checks(reinterpret_cast<const int8_t *>(16), reinterpret_cast<const int8_t *>(16), M, N, K, 128);
+  if (rc != KSD_OK) return rc;
+  if (!few_rows) return fail(KSD_EINVAL, "w8a8_gemm_few_rows: null output");
+  *few_rows = M > 0 && N > 0 && K > 0 && rows_gemm_fits(M, N, K);
+  return KSD_OK;
+}
+
 extern "C" int ksd_w8a8_gemm_nt_ex(const int8_t *a, const uint16_t *a_scales, const int8_t *w,
                                    const uint16_t *w_scales, int64_t M, int64_t N, int64_t K,
                                    int group, const float *bias, const void *residual, void *y,

@@ -9,9 +9,9 @@
 // waves takes one group, loads its slices of A and W straight into MFMA registers (they are used
 // once, so LDS staging would only add a trip) and leaves its products in LDS, where 256 threads
 // per row tile fold up to 16 groups in order. The next round's slices load during the fold.
-// Measured (device time, 16-bit output, gemm.hip's kernel -> this one): 16 x 1536 -> 1536
-// 11.2 -> 4.2 us, 128 x 1536 -> 1536 11.2 -> 7.5, 16 x 1536 -> 5888 11.1 -> 5.6, 16 x 5888 -> 1536
-// (5 K parts and their combine launch) 14.2 -> 10.9, 512 x 1536 -> 512 11.2 -> 7.7.
+// Measured (device time in a graph, 16-bit output, gemm.hip's kernel -> this one): 1 x 1536 -> 1536
+// 11.8 -> 4.4 us, 64 x 1536 -> 1536 11.8 -> 8.2, 16 x 1536 -> 4096 11.9 -> 5.1, 16 x 5888 -> 1536
+// (5 K parts and their combine launch) 15.0 -> 12.1, 512 x 1536 -> 512 11.9 -> 8.3.
 #include "ksd_common.h"
 
 namespace ksd {
@@ -162,17 +162,20 @@ static int waves(int G) {
 static int tiles(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
 }  // namespace rows
 
-// Its time grows with the row tiles that a CU works through, f = MT * ceil(workgroups / CUs), times
-// the groups: about 2.2 + 0.12 f G us, where gemm.hip's kernel takes 4.5 + 0.55 G / splits, and 4 more
-// for the combine launch of a split K. So up to f = 4, and f G = 64 where K is long enough to be split.
-// Both sides of the line (us, gemm.hip's kernel and this one): 5888 x 1536 weights, f = 4 (M = 32): 11.2,
-// 7.4; f = 8 (M = 64): 11.2, 13.4; 1536 x 5888, f G = 46 (M = 16): 14.2, 10.9; 92 (M = 32): 14.6, 14.5.
+// Its time grows with the row tiles that a CU works through, f = MT * ceil(workgroups / CUs), and the G
+// groups: about 3 us and, for each group, 0.2 at f = 1, 0.3 at f = 2, 0.4 to 0.6 at f = 4. gemm.hip's kernel
+// takes 5.2 and 0.55 G / splits, and 3 more for the combine launch of a split K. So up to f = 4, and f G = 64
+// where K is long enough to be split. At f G = 64 K is 2048, 4096 or 8192, whose rows all start in the same
+// cache channels: a full row tile's 16 of them lose there (M above 10), fewer rows and several tiles do not.
+// Both sides (us, gemm.hip's kernel and this one, M x N x K): 32 x 8192 x 1536 12.1, 8.2; 16 x 16384 x 1920
+// 14.9, 12.9; 16 x 16384 x 2048 14.1, 16.3; 16 x 6144 x 4096 14.3, 15.8; 16 x 4096 x 8192 18.0, 18.4; 8 x 8192
+// x 4096 14.9, 14.0; 64 x 4096 x 2048 13.4, 11.2; 64 x 5888 x 1536 (f = 8) 11.2, 13.4.
 // CUs are counted as 256 whatever the device has.
 bool rows_gemm_fits(int64_t M, int64_t N, int64_t K) {
   if (M > 4096) return false;
   const int mt = rows::tiles((int)M);
   const int64_t groups = K / 128, f = mt * cdiv(cdiv(N, 16) * cdiv(M, 16 * mt), 256);
-  return f <= 4 && f * groups <= 64;
+  return f <= 4 && f * groups <= (mt == 1 && M > 10 ? 63 : 64);
 }
 
 void rows_gemm(const int8_t *a, const uint16_t *as, const int8_t *w, const uint16_t *ws, int M, int N, int K,

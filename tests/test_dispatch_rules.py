@@ -21,3 +21,19 @@ def test_spine_table(fused, M, F, direct, table):
     c = ctypes.c_int(-1)
     _lib.call("ksd_ks3_spine_needs_table", M, F, fused, ctypes.byref(c))
     assert c.value == int(table < direct)
+
+
+# (rows, columns, K, the persistent kernel's time, the few-row kernel's), microseconds
+FEW_ROWS = [(1, 1536, 1536, 11.6, 4.4), (16, 16384, 1920, 14.9, 12.9), (16, 16384, 2048, 14.1, 16.3),
+            (12, 16384, 2048, 14.5, 15.4), (5, 16384, 2048, 14.1, 13.4), (16, 6144, 4096, 14.3, 15.8),
+            (8, 8192, 4096, 14.9, 14.0), (16, 8192, 3840, 15.6, 13.5), (16, 1000, 8192, 16.1, 16.9),
+            (5, 1024, 8192, 15.7, 14.6), (16, 2048, 7680, 16.6, 15.2), (32, 8192, 2048, 13.0, 12.2),
+            (64, 4096, 2048, 13.4, 11.2), (512, 512, 2048, 13.3, 11.2), (4096, 64, 2048, 13.3, 11.3),
+            (64, 5888, 1536, 11.2, 13.4)]
+
+
+@pytest.mark.parametrize("M,N,K,persistent,few", FEW_ROWS)
+def test_few_row_gemm(M, N, K, persistent, few):
+    c = ctypes.c_int(-1)
+    _lib.call("ksd_w8a8_gemm_few_rows", M, N, K, ctypes.byref(c))
+    assert c.value == int(few < persistent)
