@@ -4,19 +4,18 @@ The reference's Triton kernel fuses the down-projection GEMM, the Horner spine, 
 the per-group requantization (ks3_triton.py:100-156), following the fused kernel's own
 arithmetic contract, not the composed one.
 
-* 'int8' (NL == 2) with group 128, up to ONE_LAUNCH_MAX_ROWS rows (the eval path's
-  decode and short-prefill shapes): ksd_ks3_project_fused, one call that keeps the GEMM's
-  accumulator in its workspace and runs the fused contract on it (fp32 coordinates and LUT
-  index, no truncation, group pre-scale, second requantization). Its accumulator is the
-  unsplit ordered sum over all K groups, so it is taken only where the standalone GEMM would
-  not split K either: the outputs are then identical to the other form's. At d 1536, F 5888
-  on MI355X it takes 9 us at M = 16 and 22 at M = 256.
+* 'int8' (NL == 2) with group 128, where _one_launch_pays: ksd_ks3_project_fused. Up to 256
+  rows (decode and short prefill) it keeps the GEMM's accumulator in its workspace and runs the
+  fused contract on it (fp32 coordinates and LUT index, no truncation, group pre-scale, second
+  requantization): at d 1536, F 5888 on MI355X 9 us at M = 1 and 23 at M = 256. Past them it is
+  the reference's single-kernel form, a GEMM whose epilogue runs the contract on each finished
+  tile, with no accumulator in memory. The accumulator is the unsplit ordered sum over all K
+  groups, so the entry is taken only where the standalone GEMM would not split K either: the
+  outputs are then identical to the other form's.
 * 'int8' otherwise: ksd_w8a8_gemm_nt (fp32 accumulator out), then ksd_ks3_spine_fused, the
-  same per-element arithmetic. ``one_launch=True`` forces ksd_ks3_project_fused, which past
-  256 rows is the reference's single-kernel form: a GEMM whose epilogue runs the contract on
-  each finished tile, with no accumulator in memory, and slower for it (36.4 against 27.5 us
-  at M 512): the per-chart table (128 KB per 128-chart tile) cannot sit in LDS beside the
-  GEMM's operand ring, so the epilogue gathers it from L2.
+  same per-element arithmetic. ``one_launch`` forces either form. The single kernel gathers
+  the per-chart table (128 KB per 128-chart tile) from L2, as it cannot sit in LDS beside the
+  GEMM's operand ring.
 * 'fp16' and 'fp32' (NL == 1, 0; ks3_triton.py:76-98): ksd_ks3_spine_float on the
   accumulator (the coordinates not rounded to fp16, the warp scalars in fp16), every
   fp16/fp32 op of the Triton source rounded separately.
@@ -68,22 +67,44 @@ def project_fused(
     return hq, hs
 
 
-# Largest M for which project_fused takes ksd_ks3_project_fused by default: up to it the entry
-# keeps the accumulator in its table workspace and takes the table-free spine; past it, the GEMM
-# with its own accumulator and ksd_ks3_spine_fused is faster than the single launch (M 512:
-# 27.5 against 36.4 us, M 1024: 52.5 against 62.4).
-ONE_LAUNCH_MAX_ROWS = 256
+# Largest M for which project_fused may take ksd_ks3_project_fused by default.
+ONE_LAUNCH_MAX_ROWS = 1024
+# Largest M for which that entry is the GEMM and the table-free spine, the accumulator in its table
+# workspace (the entry's own limit: 256 values a chart); past it, the single GEMM launch.
+_ACC_ROWS = 256
 
 
 def _one_launch_pays(a_codes: torch.Tensor, w_codes: torch.Tensor) -> bool:
-    """Few rows, and a GEMM shape the standalone launch would not split along K (so both
-    forms compute the same ordered accumulator)."""
+    """Whether ksd_ks3_project_fused is the faster form, at a GEMM shape the standalone launch
+    would not split along K (so both forms compute the same ordered accumulator).
+
+    Up to 256 rows it is the same two kernels in one call. Past them it is the single launch: its
+    time goes with the rounds of 128 x 128 tiles over the CUs (256), N (the table) and K, and
+    hardly with the M N values, which the GEMM and the spine store and read, more slowly in rows
+    that are not 16-byte aligned (N % 4). The lines below are least squares over 642 shapes (M 257
+    to 1024, K 128 to 2048, N 1536 to 8192; us saved against us spent, sizes in thousands, values in
+    millions): the form they pick is within 11 percent of the faster one. Both sides (us, single and
+    two, M x K -> N): 512 x 1536 -> 5888 34, 29; 1024 x 128 -> 4096 24, 33; 1024 x 1536 -> 4096 35,
+    36; 512 x 128 -> 3001 20, 19; 1024 x 128 -> 3001 22, 29; 512 x 768 -> 5001 25, 28; 1024 x 1536
+    -> 5001 56, 52; 1024 x 768 -> 6869 53, 55; 1024 x 128 -> 6912 41, 47; 1024 x 512 -> 6912 49, 47."""
     if a_codes.dim() != 2 or w_codes.dim() != 2:
         return False
     M, K = a_codes.shape
     N = w_codes.shape[0]
     K128 = -(-K // 128) * 128
-    return 0 < M <= ONE_LAUNCH_MAX_ROWS and N > 0 and K128 > 0 and gemm_splits(M, N, K128) == 1
+    if not (0 < M <= ONE_LAUNCH_MAX_ROWS and N > 0 and K128 > 0 and gemm_splits(M, N, K128) == 1):
+        return False
+    if M <= _ACC_ROWS:
+        return True
+    rounds = -(-(-(-M // 128) * -(-N // 128)) // 256)
+    n, k, values = N / 1e3, K128 / 1e3, M * N / 1e6
+    if rounds == 1:
+        if N % 4:
+            return values * (5.4 - 0.85 * k) > 7.8 + 0.75 * n + 0.15 * k
+        return values * (5.0 - 0.8 * k) > 9.3 + 0.9 * n + 0.25 * k
+    if rounds == 2 and N % 4:
+        return values * (4.1 + 0.55 * k) > 8.4 + 2.1 * n + 4.5 * k
+    return rounds == 2 and K128 <= 256 and values > 5.6
 
 
 def _project_fused_int8(a_codes, a_scales, w_codes, w_scales, spine_codes, spine_scale,

@@ -4,8 +4,10 @@ and one is clearly the faster (CPU only: no kernel runs)."""
 import ctypes
 
 import pytest
+import torch
 
 from ksdraft_amd import _lib
+from ksdraft_amd.kernels.ks3_triton import _one_launch_pays
 
 
 # (rows, charts, time without the table, time with it), microseconds
@@ -37,3 +39,19 @@ def test_few_row_gemm(M, N, K, persistent, few):
     c = ctypes.c_int(-1)
     _lib.call("ksd_w8a8_gemm_few_rows", M, N, K, ctypes.byref(c))
     assert c.value == int(few < persistent)
+
+
+# (M, K, N, time in one launch, time of the GEMM and the spine), microseconds
+PROJECT = [(257, 128, 1536, 20.0, 11.0), (512, 1536, 5888, 34.0, 29.0),
+           (700, 1536, 5888, 57.0, 44.0), (1024, 1536, 5888, 57.0, 51.0), (600, 128, 5888, 25.0, 28.0),
+           (1024, 128, 4096, 24.0, 33.0), (1024, 512, 4096, 28.0, 35.0), (512, 512, 4096, 25.0, 21.0),
+           (1024, 128, 3001, 22.0, 29.0), (512, 128, 3001, 20.0, 18.7), (512, 768, 5001, 25.1, 28.3),
+           (700, 1792, 5001, 35.0, 38.7), (1024, 1536, 5001, 56.0, 52.0), (1024, 1792, 3001, 31.7, 33.5),
+           (1024, 768, 6869, 52.6, 54.9), (896, 512, 6869, 44.0, 48.0), (700, 1536, 6869, 57.0, 49.0),
+           (1024, 128, 6912, 41.0, 47.0), (1024, 512, 6912, 49.0, 47.0), (1025, 128, 3001, 24.0, 29.0)]
+
+
+@pytest.mark.parametrize("M,K,N,one,two", PROJECT)
+def test_one_launch_projection(M, K, N, one, two):
+    a, w = (torch.empty(r, K, dtype=torch.int8, device="meta") for r in (M, N))
+    assert _one_launch_pays(a, w) == (one < two and M <= 1024)  # never taken past 1024 rows
