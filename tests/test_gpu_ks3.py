@@ -138,13 +138,16 @@ def test_spine_fused_contract_bit_exact(M, Fn, group):
 
 
 @pytest.mark.parametrize("M,K,Fn", [(64, 128, 256), (200, 384, 130), (1, 256, 5),
-                                     (333, 1536, 1000), (130, 2048, 300), (1000, 512, 640)])
+                                     (333, 1536, 1000), (130, 2048, 300), (1000, 512, 640),
+                                     (257, 384, 130), (300, 2048, 301), (259, 256, 5), (1024, 128, 2049)])
 def test_project_fused_one_launch_bit_exact(M, K, Fn):
-    """project_fused 'int8', group 128, one_launch: the GEMM whose epilogue runs the spine
-    and both requantizations (one launch after the table) against the oracle chain, the ordered
-    sum over all K groups then the fused contract. Covers ragged M and F (partial tiles,
-    charts past F), a K that the standalone GEMM would split (2048 with 6 tiles), and
-    accumulators beyond the fp16 range (rows with large scales, clamped)."""
+    """project_fused 'int8', group 128, one_launch, against the oracle chain, the ordered sum
+    over all K groups then the fused contract: up to 256 rows the GEMM and the table-free
+    spine, past them the GEMM whose epilogue runs the spine and both requantizations (one
+    launch after the table). Covers in both ragged M and F (partial tiles, charts past F), a K
+    that the standalone GEMM would split (2048 with 6 and 9 tiles), and accumulators beyond the
+    fp16 range (rows with large scales, clamped); and a shape that takes the epilogue by
+    default."""
     cell = _random_cell(5 * M + Fn, Fn)
     rng = np.random.default_rng(M + K)
     x = rng.standard_normal((M, K)).astype(np.float32)

@@ -34,3 +34,21 @@ def test_masters_packed_in_one_launch(Fn):
         assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
     assert ki.pack_masters(co.expand(Fn, 2, 6), rs, rh) is None  # rank 2
     assert ki.pack_masters(co.half(), rs, rh) is None
+
+
+def test_masters_that_are_nan():
+    """A NaN leaves the same codes, scale bits and fp16 values as in the eleven calls."""
+    nan = float("nan")
+    co = torch.full((3, 1, 6), 0.25, device=DEV)
+    co[1, 0, 2] = nan
+    rs, rh = torch.tensor([nan, 0.5, 30.0], device=DEV), torch.tensor([0.5, nan, -2.0], device=DEV)
+    sq, ss, wsc, wss, whc, whs, sc16, sh16 = ki.pack_masters(co, rs, rh)
+    want = ki.pack_spine(co)
+    scale = quantize_last_dim((F.softplus(rs) + 1e-4).reshape(-1, 1))
+    shift = quantize_last_dim((0.5 * torch.tanh(rh)).reshape(-1, 1))
+    for a, b in ((sq, want[0]), (wsc, scale[0]), (whc, shift[0])):
+        assert torch.equal(a, b)
+    for a, b in ((ss, want[1]), (wss, scale[1]), (whs, shift[1])):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    for a, b in ((sc16, dequantize_last_dim(*scale)), (sh16, dequantize_last_dim(*shift))):
+        assert torch.allclose(a, b.reshape(-1).half(), rtol=0, atol=0, equal_nan=True)

@@ -26,9 +26,11 @@ def _spine(M, Fn, seed):
 
 
 # one row, ragged segments and row blocks, odd widths; (3700, 1984) and (3703, 1985) lie past the
-# table-free rule (7 * 2^20 values): the table readers, their row split no longer 512
-@pytest.mark.parametrize("group", [32, 128])
-@pytest.mark.parametrize("M,Fn", [(1, 1), (7, 130), (9, 128), (33, 257), (3700, 1984), (3703, 1985)])
+# table-free rule: the table readers, their row split no longer 512; the last four lie on either
+# side of it (fused and ragged rows 600 + 3.4e6 / 128-chart columns, composed 460 + 1.2e6)
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("M,Fn", [(1, 1), (7, 130), (9, 128), (33, 257), (3700, 1984), (3703, 1985),
+                                  (13881, 130), (13882, 130), (5147, 256), (5148, 256)])
 def test_spines_without_a_table(M, Fn, group):
     x, par = _spine(M, Fn, M + Fn)
     dev = [_t(p) for p in par]
