@@ -417,19 +417,25 @@ int ksd_ks3_spine_fused(const float *acc, int64_t M, int64_t F, const int8_t *sp
 int ksd_ks3_spine_needs_table(int64_t M, int64_t F, int fused, int *needed);
 
 /*
- * K8 — project_fused / _fused_gemm_spine, 'int8' mode, group 128, as one GEMM launch
- * (reference ksdraft/kernels/ks3_triton.py:100-156 and 159-195): the input-projection
- * GEMM xq . down_codes^T whose epilogue applies the spine, ReLU^2 and the per-group
- * requantization of ksd_ks3_spine_fused to each finished fp32 accumulator tile, so the
- * (M, F) accumulator never reaches memory. The accumulator is the ordered sum over all K
- * groups (K is never split). A small kernel fills the table workspace first.
+ * K8 — project_fused / _fused_gemm_spine, 'int8' mode, group 128, as one call (reference
+ * ksdraft/kernels/ks3_triton.py:100-156 and 159-195): the input-projection GEMM
+ * xq . down_codes^T, then the spine, ReLU^2 and the per-group requantization of
+ * ksd_ks3_spine_fused on its fp32 accumulator, the ordered sum over all K groups (K is never
+ * split).
+ *   M <= 256   the GEMM into the table workspace (256 values a chart), then the spine, which
+ *              evaluates its increments without a table
+ *   M > 256    a small kernel fills the table workspace with the per-chart increments, then
+ *              one GEMM launch whose epilogue applies the rest to each finished tile: the
+ *              (M, F) accumulator never reaches memory
+ * The outputs do not depend on the form.
  *   a, a_scales     (M, K) int8 codes, 16-byte aligned; (M, K/128) fp16 scales
  *   w, w_scales     (F, K) int8 down-projection codes, 16-byte aligned; (F, K/128) fp16
  *   K               a multiple of 128, > 0
  *   spine/warp buffers and tanh_lut as for ksd_ks3_spine_fwd
  *   group           128 (groups 32 and 64: ksd_w8a8_gemm_nt, then ksd_ks3_spine_fused)
  *   h_codes (M, F) int8, h_scales (M, ceil(F/128)) fp16
- *   table           workspace, (F, 256) fp32, 16-byte aligned, overwritten
+ *   table           workspace, (F, 256) fp32, 16-byte aligned, overwritten with the
+ *                   accumulator or the increments (above)
  */
 int ksd_ks3_project_fused(const int8_t *a, const uint16_t *a_scales, const int8_t *w,
                           const uint16_t *w_scales, int64_t M, int64_t F, int64_t K,

@@ -1278,6 +1278,12 @@ extern "C" int ksd_w8a8_gemm_pair(const int8_t *a0, const uint16_t *a0_scales, c
   return launch_pair(a, as, w, ws, M, N, K, y, dt, workspace, workspace_bytes, st);
 }
 
+// Few rows: the accumulator fits where the table would lie (256 fp32 values a chart), and the GEMM followed
+// by the table-free spine is the faster form (us, this after the single launch: 1 x 1536 -> 5888 27.3, 8.8;
+// 64 28.9, 17.0; 256 30.9, 23.0). The host wrapper's rule past these rows (_ACC_ROWS, kernels/ks3_triton.py)
+// rests on the same number.
+constexpr int64_t kAccRows = 256;
+
 extern "C" int ksd_ks3_project_fused(const int8_t *a, const uint16_t *a_scales, const int8_t *w,
                                      const uint16_t *w_scales, int64_t M, int64_t F, int64_t K,
                                      const int8_t *spine_codes, const uint16_t *spine_scale,
@@ -1301,10 +1307,7 @@ extern "C" int ksd_ks3_project_fused(const int8_t *a, const uint16_t *a_scales, 
   if (K == 0) return fail(KSD_EINVAL, "ks3_project_fused: K = 0 (the host wrapper handles it)");
   if ((rc = gemm_offsets_check(M, F, K, KSD_F32))) return rc;
   hipStream_t st = (hipStream_t)stream;
-  // Few rows: the accumulator fits where the table would lie (256 values a chart), and the GEMM followed by
-  // the table-free spine is the faster form (us, this after the single launch: 16 x 1536 -> 5888 27.2, 9.4;
-  // 64 29.7, 16.4; 256 33.6, 21.9).
-  if (M <= 256) {
+  if (M <= kAccRows) {
     rc = launch_o<128>(a, a_scales, w, w_scales, (int)M, (int)F, (int)K, nullptr, table, KSD_F32, st);
     if (rc != KSD_OK) return rc;
     return ks3_fused_rows(table, M, F, spine_codes, spine_scale, warp_scale, warp_shift, tanh_lut, group,

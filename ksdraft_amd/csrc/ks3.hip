@@ -1058,8 +1058,8 @@ __global__ void ks3_tanh16_kernel(const uint16_t *__restrict__ x, int64_t n, uin
 // A training forward's geometry from the fp32 masters (ks3_int8.py:262-277), one thread per chart: the
 // coefficient row's codes and scale, and the warp scalars' (softplus(raw) + 1e-4 and tanh(raw) / 2, with
 // torch's formulas and the same library functions, so the same bits) codes, scales and fp16 values. Eleven
-// launches of 4 to 5 us on 5888 values; this kernel is bound by its launch too: 55 us of
-// device time to 4.7, with the paired transposes about 20 us of the cell's 1220 at 8192 rows.
+// launches of 4 to 5 us on 5888 values; this kernel is bound by its launch too: 55 us of device time to 4.7.
+// With the paired transposes and the spine's row split the cell's pass at 8192 rows went from 1213 to 1167.
 __global__ __launch_bounds__(256) void ks3_pack_masters_kernel(
     const float *__restrict__ coeff, const float *__restrict__ raw_scale, const float *__restrict__ raw_shift,
     int64_t F, int8_t *__restrict__ spine_codes, uint16_t *__restrict__ spine_scale, int8_t *__restrict__ wsc,

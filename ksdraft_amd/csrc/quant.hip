@@ -131,7 +131,8 @@ __global__ __launch_bounds__(256) void quant_rows_fast_kernel(
 // Both operands of an int8 linear in one launch: the first nbw blocks of a row slice take the fp32
 // master W, the others x. A decode call is bound by its launches (the two quantizations of 16 x 1536
 // tokens and 1536 x 1536 weights take 2.7 and 4.3 us of device time, a launch about as long on the host):
-// that call went from 60.4 to 32.1 us with this launch, the few-row GEMM and one entry for the three.
+// that call went from 59.8 to 23.6 us with this launch, the few-row GEMM, one entry for the three and
+// cheaper bindings.
 template <int DT, int RTW, int RTX>
 __global__ __launch_bounds__(256) void quant_rows_pair_kernel(
     const float *__restrict__ w, int64_t N, int8_t *__restrict__ wcodes, uint16_t *__restrict__ wscales,
@@ -1360,6 +1361,8 @@ extern "C" int ksd_quantize_dual2(const void *x0, int64_t R0, int64_t C0, int8_t
   auto vec16 = [&](const void *x, int64_t C, const int8_t *codes) {
     return C % 8 == 0 && ((uintptr_t)x) % 16 == 0 && (C * esz) % 16 == 0 && ((uintptr_t)codes) % 8 == 0;
   };
+  // Both operands or neither: a master of 6144 x 2048 beside 64 tokens off by an element takes the ragged
+  // form too, 22.4 us (31.0 in a launch each with its own form).
   const bool vec = vec16(x0, C0, codes0) && vec16(x1, C1, codes1);
   if (!fast(R0, C0) || !fast(R1, C1) ||
       !grid_fits(cdiv(C0, 128) * cdiv(R0, 128) + cdiv(C1, 128) * cdiv(R1, 128), 512)) {

@@ -883,9 +883,10 @@ namespace ksd {
 // (uncapped, <= 64) and cap_j = min(j + 1, lmax); its key is (min(c_j, cap_j), j) and the
 // best key decides the sign. Flipping one bit changes candidate lengths in a known way:
 //   q[t - i]: c_j < i unchanged; c_j > i -> i; c_j == i -> c_j + 1 + e_j (e_j = the match
-//             run after the first mismatch). The new best is the max of the best key with
-//             c_j < i (prefix over length buckets), the latest j with c_j > i at length i,
-//             and the best extension with c_j == i (per-bucket max).
+//             run after the first mismatch). The new best is the max of the latest j with
+//             c_j > i at length i (suffix over length buckets) and the best extension with
+//             c_j == i (per-bucket max); a c_j < i never decides, as the best candidate keeps
+//             length i or is extended itself (i <= its length).
 //   k[p]:     only candidates j in [p, p + lmax) see it, at bit i = j - p: i < c_j truncates
 //             to i, i == c_j extends. A truncated key never exceeds the best key, so the sign
 //             can change only through (a) an extension beating the best (every candidate
@@ -932,7 +933,8 @@ __device__ __forceinline__ float sign_of(uint32_t key, const uint32_t *vw) {
 // Per-candidate path (scan_position): the 64 lanes of a wave split the candidates j of one
 // position t. Per-wave LDS tables for the current t (kScanMw .. words from the base):
 //   Mw[65]   best key per common-suffix length c = 0 .. 64
-//   Nw[65]   best key per c after flipping the q bit at the first mismatch
+//   Nw[65]   best key per c after flipping the q bit at the first mismatch; ~0 for the c that
+//            no q flip of this t reads (its bound is never beaten)
 //   Rk[128]  k-extension events, slot p mod 128: the best lifted key of flip k[p]
 //   tab[256] the near-run flip tables (near_flips_tables)
 constexpr int kCredWaves = 4;
@@ -1006,11 +1008,14 @@ constexpr int kCredCounters = 64;  // work counters of the balanced kernel: entr
 // the one-mismatch sets it enumerates, which is large on streams with long runs: many
 // positions with a short best match but thousands of one-mismatch candidates, or long
 // matches with long extension chains. The per-candidate path costs about the same per
-// candidate whatever the stream. The line was swept on B 4, T 2048, S 512: with mean best
-// lengths above 11, more than 30% of the positions below 8, or positions below 1024 on the
-// per-candidate path, the backward takes 5.16 / 5.85 / 5.97 ms on random streams and on
-// streams biased by 1 and 3 sigma (all positions per-candidate: 5.84 / 5.89 / 5.88; with 12,
-// 40% and 768: 5.16 / 5.88 / 6.11). A scan's cost grows with t, the bit-parallel path's hardly.
+// candidate whatever the stream, and its cost grows with t, the bit-parallel path's hardly. So
+// streams with mean best lengths above 11 or more than 30% of the positions below 8, and every
+// position below 1024, take the per-candidate path. The line was fitted at B 4, T 2048, S 512;
+// over T 500 to 2048, B S 256 to 2048 and random, biased (0.5 to 3 sigma) and run-heavy (means 3,
+// 10, 30) streams the backward is within 3% of the better single path, or faster than both
+// (the runs of mean 3 on 256 streams: 5%). ms, this rule, all positions per-candidate, all
+// bit-parallel: B 4, T 2048, S 512 random 5.18, 5.97, 6.06; biased by 1 sigma 5.87, 5.98, 15.7;
+// by 3 5.65, 5.77, 20.7; T 1500 random 3.60, 3.78, 4.47; T 1000 random 2.19, 2.18, 3.06.
 constexpr int kScanBelow = 1024;
 __device__ __forceinline__ bool cred_scan_stream(int64_t len_sum, int64_t short_cnt, int T) {
   return len_sum > 11 * (int64_t)T || 10 * short_cnt > 3 * (int64_t)T;
@@ -1210,9 +1215,8 @@ __device__ __forceinline__ void scan_position(int lane, int t, int T, int lmax, 
   // its latest j, so the bucket tables are written only when a key beats the stored one.
   // The step template flags: TOP, the first step (lanes j >= t idle, events above t - 1
   // absent), LOW, the step at j0 = 0 (caps min(j + 1, lmax) below lmax), NEAR: 0 for a step
-  // with no candidate in the near range, 1 for one that may have some, 2 to decide at run
-  // time. A lane's window words sit at a fixed offset from j0 / 32 and its funnel shift
-  // (j + 1) mod 32 is fixed.
+  // with no candidate in the near range, 1 for one that may have some. A lane's window words
+  // sit at a fixed offset from j0 / 32 and its funnel shift (j + 1) mod 32 is fixed.
   // the lane's window words kw[j0 / 32 + (lane + 1) / 32 - 2 ..], addressed from one LDS
   // address per step (kept opaque, so every step adds one offset to it)
   uint32_t kaddr = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint32_t *)(kw + ((lane + 1) >> 5) - 2);
