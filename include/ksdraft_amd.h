@@ -276,6 +276,8 @@ int ksd_embedding_gather_int8(const int8_t *codes, const uint16_t *scales, const
  * Replaces _w8a8_gemm_kernel / w8a8_gemm (reference ksdraft/kernels/gemm.py:18-50, 53-90).
  *   a (M, K) int8, a_scales (M, K/group) fp16; w (N, K) int8, w_scales (N, K/group)
  *   K must be a multiple of 128 (the host wrapper zero-pads like gemm.py:71-73).
+ *   Group 128 refuses shapes past its 32-bit tile offsets: (min(128, max(M, N)) - 1) K above
+ *   2^31 - 128, or 32 rows of y of 2^32 bytes (more than 2^31 where N is no multiple of 128).
  *   bias    NULL or (N,) fp32, added in fp32 after the group sum (linear.py:71-72)
  *   y       (M, N) of type y_dtype (KSD_F32, KSD_BF16, KSD_F16, KSD_F16_SAT)
  */
